@@ -14,13 +14,13 @@ namespace nat {
 // so stream-only followed by this pass equals a fused step bit for bit. INIT: the
 // reference's initialisation collision (velocity read from the stored field).
 template <int Q, typename T, bool INIT>
-__global__ __launch_bounds__(256) void k_collide(T* f, int64_t stride, int64_t n, CollideArgs<T> ca) {
+__global__ __launch_bounds__(256) void k_collide(T* f, int64_t stride, int64_t n, CollideArgs<T> ca, int macro) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   T fs[Q];
 #pragma unroll
   for (int q = 0; q < Q; q++) fs[q] = f[(int64_t)q * stride + i];
-  bgk_collide_store_pairs<Q, T, INIT>(fs, ca, i, true, f, stride);
+  bgk_collide_store_pairs<Q, T, INIT>(fs, ca, i, macro != 0, f, stride);
 }
 
 // The pseudo-entropic stabilizer as a pass of its own (PseudoEntropicStabilizer::apply,
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(SUM_BS) void k_sums_final(const double* __restrict_
 }  // namespace nat
 
 template <typename T>
-static int launch_collide_typed(nat_ctx* ctx, bool init) {
+static int launch_collide_typed(nat_ctx* ctx, bool init, bool stab, bool macro) {
   using namespace nat;
   const int bs = 256;
   const unsigned grid = (unsigned)((ctx->n_store + bs - 1) / bs);
@@ -196,16 +196,16 @@ static int launch_collide_typed(nat_ctx* ctx, bool init) {
   ca.u = (T*)ctx->u;
   ca.mstride = ctx->n_store;
   ca.status = ctx->d_status;
-  ca.stab = 0;
+  ca.stab = stab ? 1 : 0;
   T* f = (T*)ctx->f[ctx->cur];
 #define NAT_KC(QQ)                                                                                              \
   if (ctx->Q == QQ) {                                                                                          \
     if (init)                                                                                                  \
       hipLaunchKernelGGL((k_collide<QQ, T, true>), dim3(grid), dim3(bs), 0, ctx->stream, f, ctx->stride,       \
-                         ctx->n_store, ca);                                                                    \
+                         ctx->n_store, ca, (int)macro);                                                                    \
     else                                                                                                       \
       hipLaunchKernelGGL((k_collide<QQ, T, false>), dim3(grid), dim3(bs), 0, ctx->stream, f, ctx->stride,      \
-                         ctx->n_store, ca);                                                                    \
+                         ctx->n_store, ca, (int)macro);                                                                    \
     NAT_HIP(hipGetLastError());                                                                                \
     return 0;                                                                                                  \
   }
@@ -218,7 +218,16 @@ static int launch_collide_typed(nat_ctx* ctx, bool init) {
 }
 
 int nat_launch_collide(nat_ctx* ctx, int init) {
-  return ctx->fp32 ? launch_collide_typed<float>(ctx, init != 0) : launch_collide_typed<double>(ctx, init != 0);
+  return ctx->fp32 ? launch_collide_typed<float>(ctx, init != 0, false, true)
+                   : launch_collide_typed<double>(ctx, init != 0, false, true);
+}
+
+// The collision that ends a run of collide-then-stream launches: with the stabilizer where the
+// context has it on, as every collision inside nat_step, and the fields when macro.
+int nat_launch_collide_step(nat_ctx* ctx, bool macro) {
+  const bool stab = ctx->stab_on() != 0;
+  return ctx->fp32 ? launch_collide_typed<float>(ctx, false, stab, macro)
+                   : launch_collide_typed<double>(ctx, false, stab, macro);
 }
 
 int nat_launch_stabilize(nat_ctx* ctx) {

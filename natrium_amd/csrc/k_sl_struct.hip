@@ -31,6 +31,10 @@
 // between passes). With FP32 storage the populations are shifted,
 // f~ = f - w rho0, so only perturbations are rounded to FP32.
 //
+// Runs of several steps at p = 2-4 take the collide-then-stream form of k_sl_push.hip where it is
+// faster; this kernel serves single steps, packed steps, p = 1 and 6, unequal axes and the large
+// FP64 boxes. Both give the same populations bit for bit.
+//
 // Storage: unique periodic nodes (N_a p per axis, x fastest); the FE_Q DoFs on the
 // upper periodic faces are copies of the lower ones and are produced at download.
 #include <map>

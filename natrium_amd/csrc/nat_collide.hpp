@@ -103,18 +103,18 @@ constexpr int opposite(int i) {
 }
 
 // FP64 BGK collision of populations held in storage precision, every relaxed population
-// stored as soon as it is formed. The equilibrium of each opposite pair (i, i') comes from
-// shared even and odd parts: f_eq(i/i') = w (E +- O), E = drho + rho (ue^2/2 - 3u.u/2),
+// handed to store(std::integral_constant<int, i>, value) as soon as it is formed. The
+// equilibrium of each opposite pair (i, i') comes from shared even and odd parts: f_eq(i/i') = w (E +- O), E = drho + rho (ue^2/2 - 3u.u/2),
 // O = rho ue (the direction-by-direction form of Equilibria.h:66-83 up to FP64 rounding).
 // Every step kernel and the collision-only pass use this one function, so their results
-// agree bit for bit. Stores go through a uniform direction base and a 32-bit byte offset.
+// agree bit for bit.
 //
 // INIT: the collision of the reference's iterative initialisation
 // (collision_advanced/CollisionOperator.h:79-91, inInitializationProcedure): the velocity
 // is read from the stored field (u / scaling) instead of computed, and only rho is written.
-template <int Q, typename T, bool INIT = false>
-__device__ __forceinline__ void bgk_collide_store_pairs(const T (&f)[Q], const CollideArgs<T>& ca, int64_t node,
-                                                        bool write_macro, T* __restrict__ fout, int64_t stride) {
+template <int Q, typename T, bool INIT, typename F>
+__device__ __forceinline__ void bgk_collide_pairs(const T (&f)[Q], const CollideArgs<T>& ca, int64_t node,
+                                                  bool write_macro, F&& store) {
   // Fused multiply-adds are written out and no other contraction is allowed: every kernel
   // that inlines this function rounds the same way, whatever the compiler decides elsewhere.
 #pragma clang fp contract(off)
@@ -153,29 +153,11 @@ __device__ __forceinline__ void bgk_collide_store_pairs(const T (&f)[Q], const C
   const double base = fma(-rho, 1.5 * uu, drho);  // even part without the ue^2 term
   const double hr = 0.5 * rho;
   const double om = ca.omega64;
-  const uint32_t nb = (uint32_t)node * (uint32_t)sizeof(T);
-  // raw buffer stores against a uniform direction base with the sc1 cache policy
-  // (device-scope write-through): the step's output reaches memory while the kernel
-  // runs instead of in the write-back at the kernel boundary (measured 1.8% on the
-  // 16^3 p=4 D3Q27 step in FP32, 3% in FP64). Offsets stay below 2^31: the launcher
-  // checks one direction's array against INT32_MAX bytes.
-  auto store = [&](int i, double v) {
-    const uint64_t pb = (uint64_t)(fout + (int64_t)i * stride);
-    const uint32_t phi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(pb >> 32));
-    const uint32_t plo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)pb);
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(((uint64_t)phi << 32) | (uint64_t)plo), (short)0, 0x7fffffff, 0x00020000);
-    if constexpr (sizeof(T) == 4)
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (float)v), rs, (int)nb, 0, 16);
-    else
-      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(unsigned __attribute__((ext_vector_type(2))), v), rs,
-                                            (int)nb, 0, 16);
-  };
   if ((Q == 9 || Q == 19) && ca.stab) {
     // stabilized: f_eq + (1 - omega) P f_neq; the correction is even in e
     double uu3[3] = {u[0], u[1], D == 3 ? u[2] : 0.0};
     const StabPi<Q> pn = stab_neq<Q>(stab_moments<Q>(fd), drho, rho, uu3, om);
-    store(0, fma(L::w[0], base, stab_term<Q>(pn, 0)));
+    store(std::integral_constant<int, 0>{}, fma(L::w[0], base, stab_term<Q>(pn, 0)));
     static_for<1, Q>([&](auto I) {
       constexpr int i = decltype(I)::value;
       constexpr int o = opposite<Q>(i);
@@ -189,12 +171,12 @@ __device__ __forceinline__ void bgk_collide_store_pairs(const T (&f)[Q], const C
         const double E = fma(hr, ue * ue, base);
         const double O = rho * ue;
         const double wE = fma(L::w[i], E, stab_term<Q>(pn, i)), wO = L::w[i] * O;
-        store(i, wE + wO);
-        store(o, wE - wO);
+        store(I, wE + wO);
+        store(std::integral_constant<int, o>{}, wE - wO);
       }
     });
   } else {
-    store(0, fma(-om, fd[0] - L::w[0] * base, fd[0]));
+    store(std::integral_constant<int, 0>{}, fma(-om, fd[0] - L::w[0] * base, fd[0]));
     static_for<1, Q>([&](auto I) {
       constexpr int i = decltype(I)::value;
       constexpr int o = opposite<Q>(i);
@@ -208,8 +190,8 @@ __device__ __forceinline__ void bgk_collide_store_pairs(const T (&f)[Q], const C
         const double E = fma(hr, ue * ue, base);
         const double O = rho * ue;
         const double wE = L::w[i] * E, wO = L::w[i] * O;
-        store(i, fma(-om, fd[i] - (wE + wO), fd[i]));
-        store(o, fma(-om, fd[o] - (wE - wO), fd[o]));
+        store(I, fma(-om, fd[i] - (wE + wO), fd[i]));
+        store(std::integral_constant<int, o>{}, fma(-om, fd[o] - (wE - wO), fd[o]));
       }
     });
   }
@@ -220,6 +202,32 @@ __device__ __forceinline__ void bgk_collide_store_pairs(const T (&f)[Q], const C
       for (int d = 0; d < D; d++) ca.u[d * ca.mstride + node] = (T)(u[d] * ca.scaling);
     }
   }
+}
+
+// The collision with every relaxed population stored to fout through a uniform direction base
+// and a 32-bit byte offset.
+template <int Q, typename T, bool INIT = false>
+__device__ __forceinline__ void bgk_collide_store_pairs(const T (&f)[Q], const CollideArgs<T>& ca, int64_t node,
+                                                        bool write_macro, T* __restrict__ fout, int64_t stride) {
+  const uint32_t nb = (uint32_t)node * (uint32_t)sizeof(T);
+  // raw buffer stores against a uniform direction base with the sc1 cache policy
+  // (device-scope write-through): the step's output reaches memory while the kernel
+  // runs instead of in the write-back at the kernel boundary (measured 1.8% on the
+  // 16^3 p=4 D3Q27 step in FP32, 3% in FP64). Offsets stay below 2^31: the launcher
+  // checks one direction's array against INT32_MAX bytes.
+  auto store = [&](auto I, double v) {
+    const uint64_t pb = (uint64_t)(fout + (int64_t)decltype(I)::value * stride);
+    const uint32_t phi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(pb >> 32));
+    const uint32_t plo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)pb);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(((uint64_t)phi << 32) | (uint64_t)plo), (short)0, 0x7fffffff, 0x00020000);
+    if constexpr (sizeof(T) == 4)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (float)v), rs, (int)nb, 0, 16);
+    else
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(unsigned __attribute__((ext_vector_type(2))), v), rs,
+                                            (int)nb, 0, 16);
+  };
+  bgk_collide_pairs<Q, T, INIT>(f, ca, node, write_macro, store);
 }
 
 }  // namespace nat
