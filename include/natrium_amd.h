@@ -232,17 +232,17 @@ int nat_step_packed(nat_ctx* const* ctxs, int n, int nsteps);
  * timing launches write only the idle population buffer: populations, fields and time are
  * unchanged, and results do not depend on the shape. SL contexts (not compressible):
  *   structured backend: the tiles; tile receives the chosen (x, y, z) extents;
- *   general backend: with FP32 storage in 3D the six-wave form and the DEEP form (4 waves,
- *     more source rows and the next departure record in flight; by default chosen when its
- *     grid fits one round of the device); tile receives the chosen form's (DoFs per block,
- *     waves per SIMD it is built for, z-planes of source rows loaded together). */
+ *   general backend: with FP32 storage in 3D the eight-wave and the sixteen-wave form of a block
+ *     of DoFs (the latter by default up to 5/2 blocks per CU); tile receives the chosen form's
+ *     (DoFs per block, waves per SIMD it is built for, z-planes of source rows loaded
+ *     together). */
 int nat_autotune(nat_ctx* ctx, int nsteps, int* tile /* 3, may be NULL */);
 
 /* Pins the general SL backend's kernel form, no counterpart in the reference: form -1 the
- * default rule (DEEP when its grid fits one round of the device), 0 the six-wave form, 1 the
- * DEEP form (FP32 storage in 3D; other contexts have one form and accept only -1 and 0). Both
- * forms give bit-identical results; the choice only moves the step time. NAT_ERR_ARG for
- * another value or backend. */
+ * default rule (sixteen waves per block of DoFs up to 5/2 blocks per CU, else eight), 0 eight
+ * waves, 1 sixteen (FP32 storage in 3D; other contexts follow the default rule and accept only
+ * -1 and 0). Both forms give bit-identical results; the choice only moves the step time.
+ * NAT_ERR_ARG for another value or backend. */
 int nat_set_general_form(nat_ctx* ctx, int form);
 
 /* ---- Output and restart (host side, from fields downloaded through this API) ---- */

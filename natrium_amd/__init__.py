@@ -394,7 +394,7 @@ class Solver:
 
     def set_general_form(self, form):
         """Pin the general backend's kernel form (nat_set_general_form): -1 default rule,
-        0 six-wave form, 1 DEEP form (FP32 storage, 3D)."""
+        0 eight waves per block, 1 sixteen waves per block (FP32 storage, 3D)."""
         self._check(lib().nat_set_general_form(self._h, int(form)))
 
 

@@ -56,52 +56,63 @@ struct GeneralArgs {
   double dgl[MAXP + 1][MAXP + 1];  // x_a - x_k
 };
 
-// Launch shape. The direction loop is bound by the latency of its gathers, so the
-// kernel wants many waves per SIMD; holding the Q streamed populations in registers
-// across that loop forces either few waves or scratch spills. Where Q populations of
-// a block fit in LDS at >= 4 waves per SIMD (FP32 storage; FP64 up to Q = 19), each
-// thread parks its populations in its own LDS column (no barrier: no thread reads
-// another's column), the direction loop stays rolled, and the collision reloads the
-// column. FP32: 6 waves (80 registers); FP64: the 4 waves its LDS allows. FP64 D3Q27
-// (216 B per DoF) keeps the populations in registers at 6 waves. On 24^3 perturbed
-// cells, p = 3, this shape gives D3Q19 FP32 1.25 -> 1.58 and D3Q27 FP32 0.86 -> 1.25
-// GLUPS over the unrolled register form.
+// Launch shape. A block owns G groups of 64 DoFs and has W waves; the items (group, direction)
+// are dealt to the waves direction by direction, each wave taking another group from one
+// direction to the next, and the streamed populations meet in LDS before one wave per group
+// collides it. Two things follow. Waves whose DoFs lie on the faces of the box spend several
+// times as long on a direction (kept_wave), and the block shares that. And W may exceed G, so
+// that a mesh of few blocks still has waves to hide its dependent loads behind: one HBM round
+// trip (the record) and P + 1 L2 round trips (the source planes) per item.
 //
-// Within one direction the rows of `zu` z-planes of the source block are loaded
-// together: one plane at 80 registers, as many planes as keep the raw rows within 64
-// registers at 4 waves (C3 FP64, two planes: 358 -> 342 us per step). The DEEP form of
-// the FP32 3D kernel runs at 4 waves with those planes in flight and the next
-// direction's record prefetched; it is launched when the grid fits one round of it,
-// where each wave's dependent loads, not the number of waves, set the time (D3Q27 p = 3
-// on 16^3 perturbed cells, 460 blocks: 219 us per step in the 6-wave form, 118 in the
-// DEEP one). A grid that fills the 6-wave form (C3: 1520 blocks) keeps that form (179 us
-// against 194 for the 4-wave one).
-template <int D, int Q, int P, typename T, bool DEEP>
+// Two forms. WIDE: W = 16 (8 at p >= 5, for registers), for grids of few blocks. Otherwise
+// W = 2 G; FP32 storage at 6 waves per SIMD (80 registers), FP64 with the registers one plane of
+// rows in flight needs (more waves, or more rows, measured slower: they take the L1 and L2 lines
+// of the others' source planes). Before, a thread took its DoF through all directions by itself.
+// us per step, perturbed boxes, before / W = 2 G / wide (the rule's choice in [ ]):
+//   D3Q19 p=3 FP32   6^3 cells  64.0/ 34.3/[24.4]   16^3  91.8/ 45.3/[44.5]   24^3 157/[100]/111   36^3 511/[364]
+//             FP64   6^3        70.1/ 59.4/[25.7]   16^3  90.6/[63.9]/74.9    24^3 241/[179]/237   36^3 676/[602]
+//   D3Q27 p=3 FP32  10^3        71.3/ 38.9/[29.5]   24^3   242/[127]/143      30^3 542/[281]
+//             FP64  10^3        90.2/ 66.4/[31.9]   24^3   333/[259]/361      30^3 638/[504]
+//   D3Q19 p=2 FP64  16^3        48.0/ 24.7/[20.3]   36^3   170/[135]/139
+//   D2Q9  p=4 FP64  32^2 walls  20.8/    -/[ 9.5]   64^2  23.7/ 18.3/[14.7]   128^2 43.6/[31.9]/36.8
+template <int D, int Q, int P, typename T, bool WIDE>
 struct GeneralShape {
-  static constexpr bool lds = sizeof(T) == 4 || Q * 8 <= 160;
-  static constexpr int waves = DEEP ? 4 : (sizeof(T) == 4 ? 6 : (lds ? 4 : 6));
-  // DoFs per block: 128 with FP64 storage (C3 FP64 +6% over 256), 256 with FP32
-  // (128 measured 18% slower on D3Q27)
-  static constexpr int bs = sizeof(T) == 8 ? 128 : 256;
+  static constexpr int G = sizeof(T) == 4 ? 4 : 2;
+  static constexpr int W = WIDE ? (P >= 5 ? 8 : 16) : 2 * G;
+  static constexpr int bs = G * 64;  // DoFs per block
+  static constexpr int nt = W * 64;
+  static constexpr int waves = WIDE ? (P >= 5 ? 2 : 4) : (sizeof(T) == 4 ? 6 : 2);  // per SIMD, at least
+  // source rows of `zu` z-planes are loaded together, as their raw values fit 64 registers
   static constexpr int nz = D == 3 ? P + 1 : 1;
   static constexpr int plane_regs = (P + 1) * (P + 1) * (int)(sizeof(T) / 4);
   static constexpr int zfit = 64 / plane_regs < 1 ? 1 : (64 / plane_regs > nz ? nz : 64 / plane_regs);
-  static constexpr int zu = (waves == 4 && lds) ? zfit : 1;
-  // the next direction's record loaded before this direction's gathers (FP32 at 6 waves:
-  // spills and loses 14%)
-  static constexpr bool prefetch = sizeof(T) == 8 || DEEP;
+  static constexpr int zu = WIDE ? zfit : 1;
+  // the next item's record loaded before this item's gathers (at 6 waves: spills, 108 -> 123 us)
+  static constexpr bool prefetch = waves < 6;
+  // cut-off rows a wave sums together, at most 4, by the LDS that keeps the waves resident
+  static constexpr int NL = D == 3 ? (P + 1) * (P + 1) * (P + 1) : (P + 1) * (P + 1);
+  static constexpr int row_bytes = (NL + 3 * (P + 1)) * 8;
+  static constexpr int spare = (WIDE ? 80 * 1024 : 160 * 1024 * W / (4 * waves) - 64) -
+                               (Q - 1) * bs * (int)sizeof(T) - bs * 4 - (P + 1) * (P + 1) * 8;
+  static constexpr int fit = spare / (W * row_bytes);
+  static constexpr int R = fit < 0 ? 0 : (fit > 4 ? 4 : fit);
 };
 
-// Lagrange values at x_a + d (anchor a), in FP64: prod_{k != j} (x_a - x_k + d) / den_j
+// Lagrange values at x_a + d (anchor a), in FP64: prod_{k != j} (x_a - x_k + d) / den_j.
+// The differences come from an LDS copy of the table: the anchor differs from lane to lane, and
+// from the kernel arguments its row is six gathers per direction, behind the record's load.
 template <int P>
-__device__ __forceinline__ void basis_at(const double (&dgl)[MAXP + 1][MAXP + 1], const double (&inv)[MAXP + 1],
-                                         int a, double d, double (&v)[P + 1]) {
+__device__ __forceinline__ void basis_at(const double* dgl, const double (&inv)[MAXP + 1], int a, double d,
+                                         double (&v)[P + 1]) {
+  double s[P + 1];
+#pragma unroll
+  for (int k = 0; k <= P; k++) s[k] = dgl[a * (P + 1) + k] + d;
 #pragma unroll
   for (int j = 0; j <= P; j++) {
     double t = inv[j];
 #pragma unroll
     for (int k = 0; k <= P; k++)
-      if (k != j) t *= (dgl[a][k] + d);
+      if (k != j) t *= s[k];
     v[j] = t;
   }
 }
@@ -120,40 +131,42 @@ __device__ __forceinline__ void basis_xi(const double (&x)[MAXP + 1], const doub
 }
 
 // p+1 consecutive lattice values (one x row of a source cell) through raw buffer
-// loads: byte offsets against a per-direction resource, 16-byte loads where the row
-// length allows (buffer loads need dword alignment only).
+// loads: byte offsets against a per-direction resource, in the fewest loads the row's
+// length allows (16, 12, 8 and 4 bytes; buffer loads need dword alignment only): p = 2
+// rows are one load in FP32 and two in FP64, p = 4 rows two and three.
 template <int P, typename T>
 __device__ __forceinline__ void load_row(__amdgpu_buffer_rsrc_t r, int off, double (&v)[P + 1]) {
-  if constexpr (sizeof(T) == 4 && (P + 1) % 4 == 0) {
-#pragma unroll
-    for (int q = 0; q < (P + 1) / 4; q++) {
-      const auto x = __builtin_amdgcn_raw_buffer_load_b128(r, off + 16 * q, 0, 0);
-#pragma unroll
-      for (int k = 0; k < 4; k++) v[4 * q + k] = (double)__builtin_bit_cast(float, (unsigned)x[k]);
+  constexpr int W = (int)sizeof(T) / 4, ND = (P + 1) * W;  // dwords per value and per row
+  unsigned q[ND];
+  static_for<0, (ND + 3) / 4>([&](auto K) {
+    constexpr int k = 4 * decltype(K)::value, n = ND - k < 4 ? ND - k : 4;
+    if constexpr (n == 4) {
+      const auto x = __builtin_amdgcn_raw_buffer_load_b128(r, off + 4 * k, 0, 0);
+      static_for<0, 4>([&](auto J) { q[k + decltype(J)::value] = x[decltype(J)::value]; });
+    } else if constexpr (n == 3) {
+      const auto x = __builtin_amdgcn_raw_buffer_load_b96(r, off + 4 * k, 0, 0);
+      static_for<0, 3>([&](auto J) { q[k + decltype(J)::value] = x[decltype(J)::value]; });
+    } else if constexpr (n == 2) {
+      const auto x = __builtin_amdgcn_raw_buffer_load_b64(r, off + 4 * k, 0, 0);
+      static_for<0, 2>([&](auto J) { q[k + decltype(J)::value] = x[decltype(J)::value]; });
+    } else {
+      q[k] = __builtin_amdgcn_raw_buffer_load_b32(r, off + 4 * k, 0, 0);
     }
-  } else if constexpr (sizeof(T) == 4 && (P + 1) % 2 == 0) {
+  });
 #pragma unroll
-    for (int q = 0; q < (P + 1) / 2; q++) {
-      const auto x = __builtin_amdgcn_raw_buffer_load_b64(r, off + 8 * q, 0, 0);
-      v[2 * q] = (double)__builtin_bit_cast(float, (unsigned)x[0]);
-      v[2 * q + 1] = (double)__builtin_bit_cast(float, (unsigned)x[1]);
-    }
-  } else if constexpr (sizeof(T) == 8 && (P + 1) % 2 == 0) {
-#pragma unroll
-    for (int q = 0; q < (P + 1) / 2; q++) {
-      const auto x = __builtin_amdgcn_raw_buffer_load_b128(r, off + 16 * q, 0, 0);
-      v[2 * q] = __builtin_bit_cast(double, ((unsigned long)(unsigned)x[1] << 32) | (unsigned)x[0]);
-      v[2 * q + 1] = __builtin_bit_cast(double, ((unsigned long)(unsigned)x[3] << 32) | (unsigned)x[2]);
-    }
-  } else {
-#pragma unroll
-    for (int m = 0; m <= P; m++) {
-      if constexpr (sizeof(T) == 4)
-        v[m] = (double)__builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off + 4 * m, 0, 0));
-      else
-        v[m] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off + 8 * m, 0, 0));
-    }
+  for (int m = 0; m <= P; m++) {
+    if constexpr (W == 1)
+      v[m] = (double)__builtin_bit_cast(float, q[m]);
+    else
+      v[m] = __builtin_bit_cast(double, ((unsigned long)q[2 * m + 1] << 32) | q[2 * m]);
   }
+}
+
+// min(|a|, |b|) in one instruction (fmin of fabs also quiets signalling NaNs, two more)
+__device__ __forceinline__ double min_abs(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+  return r;
 }
 
 // Weights, cut-off and arithmetic in FP64 for both storage precisions (FP32 weights
@@ -204,8 +217,8 @@ __device__ __forceinline__ DepRec<D, T> load_rec(const GeneralArgs<T>& a, int64_
 // 1-D Lagrange weights of a departure record in FP64 and the lattice index of its cell's
 // first node (records with rec.c >= 0 only).
 template <int D, int P, typename T>
-__device__ __forceinline__ int64_t dep_weights(const GeneralArgs<T>& a, const DepRec<D, T>& rec, double (&lx)[P + 1],
-                                               double (&ly)[P + 1], double (&lz)[P + 1]) {
+__device__ __forceinline__ int64_t dep_weights(const GeneralArgs<T>& a, const double* dgl, const DepRec<D, T>& rec,
+                                               double (&lx)[P + 1], double (&ly)[P + 1], double (&lz)[P + 1]) {
   constexpr int NP = P + 1;
   constexpr int NL = (D == 3) ? NP * NP * NP : NP * NP;
   int c;
@@ -220,9 +233,9 @@ __device__ __forceinline__ int64_t dep_weights(const GeneralArgs<T>& a, const De
     const int lin = code - c * NL;
     const int ax = lin % NP, ay = (lin / NP) % NP, az = (D == 3) ? lin / (NP * NP) : 0;
     constexpr double q = 1.0 / 1073741824.0;
-    basis_at<P>(a.dgl, a.inv_den, ax, (double)rec.off[0] * q, lx);
-    basis_at<P>(a.dgl, a.inv_den, ay, (double)rec.off[1] * q, ly);
-    if constexpr (D == 3) basis_at<P>(a.dgl, a.inv_den, az, (double)rec.off[2] * q, lz);
+    basis_at<P>(dgl, a.inv_den, ax, (double)rec.off[0] * q, lx);
+    basis_at<P>(dgl, a.inv_den, ay, (double)rec.off[1] * q, ly);
+    if constexpr (D == 3) basis_at<P>(dgl, a.inv_den, az, (double)rec.off[2] * q, lz);
   }
   const uint32_t q0 = a.divN0.div((uint32_t)c), q1 = a.divN1.div(q0);
   const int cx = c - (int)q0 * a.N[0];
@@ -253,97 +266,175 @@ __device__ __forceinline__ double kept_sum(__amdgpu_buffer_rsrc_t rs, int b0, in
   double kept = 0;
 #pragma unroll 1
   for (int mz = 0; mz < NZ; mz++) {
+    // a departure point on a node line has exactly one non-zero weight there: the other lines'
+    // rows add nothing
+    if (D == 3 && !__any(lz[mz] != 0.0)) continue;
+    // a plane's rows together at p <= 3, one row at a time above (registers)
+    constexpr int NV = P <= 3 ? NP : 1;
 #pragma unroll 1
-    for (int my = 0; my <= P; my++) {
-      double v[NP];
-      load_row<P, T>(rs, b0 + (int)sizeof(T) * (n0 * (my + n1 * mz)), v);
+    for (int m0 = 0; m0 < NP; m0 += NV) {
+      double v[NV][NP];
 #pragma unroll
-      for (int mx = 0; mx <= P; mx++) {
-        const double w = (D == 3) ? lx[mx] * ly[my] * lz[mz] : lx[mx] * ly[my];
-        kept += fabs(w) < 1e-10 ? 0.0 : w * v[mx];
+      for (int m = 0; m < NV; m++) load_row<P, T>(rs, b0 + (int)sizeof(T) * (n0 * (m0 + m + n1 * mz)), v[m]);
+#pragma unroll
+      for (int m = 0; m < NV; m++) {
+        const int my = NV == NP ? m : m0;
+        if (!__any(ly[my] != 0.0)) continue;
+#pragma unroll
+        for (int mx = 0; mx <= P; mx++) {
+          const double w = (D == 3) ? lx[mx] * ly[my] * lz[mz] : lx[mx] * ly[my];
+          kept += fabs(w) < 1e-10 ? 0.0 : w * v[m][mx];
+        }
       }
     }
   }
   return kept;
 }
 
+// The cut-off rows of a wave, a few lanes' rows at a time and a term per lane: each lane with a
+// cut-off row (cut) puts its weights into LDS, all lanes form one product each of that row (one
+// gather for the whole (p+1)^D stencil), and the row's lane adds the products up in the order and
+// with the roundings of kept_sum. Perturbed cells give almost every wave such a lane in the six
+// directions along the axes (24^3 cells, p = 3: two of the three weight factors are then of the
+// order of the distortion), and the serial sum costs the whole wave 16 row loads and
+// about 900 VALU instructions each time (24^3 cells, p = 3, D3Q19 FP32: 150 -> 135 us per step).
+// sc: the wave's R x (3 (P + 1) + NL) doubles of LDS. Waves with more than R such lanes keep the
+// serial sum: a whole wave of them costs it no more than one.
+template <int D, int P, typename T, int R>
+__device__ __forceinline__ double kept_wave(__amdgpu_buffer_rsrc_t rs, bool cut, int b0, int n0, int n1,
+                                            const double (&lx)[P + 1], const double (&ly)[P + 1],
+                                            const double (&lz)[P + 1], double acc, double* sc) {
+  constexpr int NP = P + 1, NL = (D == 3) ? NP * NP * NP : NP * NP, WS = D * NP;
+  const unsigned long long m = __ballot(cut);
+  const int count = __popcll(m);
+  if (R == 0 || count > R) {
+    if (cut) acc = kept_sum<D, P, T>(rs, b0, n0, n1, lx, ly, lz);
+    return acc;
+  }
+  const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  const int slot = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+  double* const prod = sc + R * WS;
+  if (cut) {
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
+      sc[slot * WS + k] = lx[k];
+      sc[slot * WS + NP + k] = ly[k];
+      if constexpr (D == 3) sc[slot * WS + 2 * NP + k] = lz[k];
+    }
+  }
+  asm volatile("" ::: "memory");  // one wave's LDS operations complete in order; the compiler keeps it
+#pragma unroll
+  for (int c = 0; c < (NL + 63) / 64; c++) {
+    const int t = c * 64 + lane;
+    const int mx = t % NP, my = (t / NP) % NP, mz = D == 3 ? t / (NP * NP) : 0;
+    const int off = (int)sizeof(T) * (mx + n0 * (my + n1 * mz));
+    unsigned long long left = m;
+    T v[R > 0 ? R : 1];
+#pragma unroll
+    for (int s = 0; s < R; s++) {
+      const int b = __builtin_amdgcn_readlane(b0, left ? __builtin_ctzll(left) : 0);
+      if (left && t < NL) {
+        if constexpr (sizeof(T) == 4)
+          v[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, b + off, 0, 0));
+        else
+          v[s] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, b + off, 0, 0));
+      }
+      left &= left - 1;
+    }
+#pragma unroll
+    for (int s = 0; s < R; s++) {
+      if (s < count && t < NL) {
+        const double wxy = sc[s * WS + mx] * sc[s * WS + NP + my];
+        const double w = (D == 3) ? wxy * sc[s * WS + 2 * NP + mz] : wxy;
+        prod[s * NL + t] = fabs(w) < 1e-10 ? 0.0 : w * (double)v[s];
+      }
+    }
+  }
+  asm volatile("" ::: "memory");
+  if (cut) {
+    double kept = 0;
+#pragma unroll 16
+    for (int t = 0; t < NL; t++) kept += prod[slot * NL + t];
+    acc = kept;
+  }
+  asm volatile("" ::: "memory");
+  return acc;
+}
+
 // Returns the streamed population of direction al at DoF i from its departure record.
 //
 // Reference cut-off: product weights |w| < 1e-10 are dropped. When the product of the
 // smallest 1-D magnitudes is >= 1e-10 no product can fall under it and the sum factorises
-// row by row (rows through 16-, 8- or 4-byte buffer loads). Otherwise (a departure point
-// on a node line of some axis, as for DoFs on the box faces, which almost every 64-DoF wave
-// holds) the lane sums the kept terms again, one product at a time, with the source rows
-// re-read one at a time (a compact loop: the whole wave runs it when one lane needs it, so
-// it must not raise the register count of the direction loop). Lanes reflected at a wall
-// (another direction's array) gather term by term.
-template <int D, int Q, int P, typename T, int ZU>
-__device__ __forceinline__ T gen_direction(const GeneralArgs<T>& a, int64_t i, int al, int widx, unsigned wmask,
-                                           const DepRec<D, T>& rec) {
+// row by row (rows through buffer loads). Otherwise (a departure point on or next to a node
+// line of some axis) the kept terms are summed one product at a time (kept_wave). Lanes
+// reflected at a wall (another direction's array) gather term by term. The fused
+// multiply-adds of the factorised sum are written out, so all forms of the kernel agree
+// bit for bit.
+template <int D, int Q, int P, typename T, int ZU, int R>
+__device__ __forceinline__ T gen_direction(const GeneralArgs<T>& a, const double* dgl, double* sc, int64_t i, int al,
+                                           int widx, unsigned wmask, const DepRec<D, T>& rec) {
+#pragma clang fp contract(off)
   constexpr int NP = P + 1;
   const int n0 = a.nfe[0], n1 = a.nfe[1];
   const T* own = a.fin + (int64_t)al * a.stride;
   const bool flip = (wmask >> al) & 1u;
-  const T* src = flip ? a.fin + (int64_t)opposite<Q>(al) * a.stride : own;
   const double bias = widx >= 0 ? a.wall_bias[(int64_t)widx * Q + al] : 0.0;
-  if (rec.c < 0) return (T)((double)own[i] + bias);  // tracker life-time limit: identity row
+  const __amdgpu_buffer_rsrc_t rs = dir_rsrc<T>(a, own);
   double lx[NP], ly[NP], lz[NP];
-  const int64_t base = dep_weights<D, P, T>(a, rec, lx, ly, lz);
   double acc = 0;
-  double mn = 1;
-  {
-    double mx_ = fabs(lx[0]), my_ = fabs(ly[0]), mz_ = (D == 3) ? fabs(lz[0]) : 1.0;
-#pragma unroll
-    for (int m = 1; m <= P; m++) {
-      mx_ = fmin(mx_, fabs(lx[m]));
-      my_ = fmin(my_, fabs(ly[m]));
-      if constexpr (D == 3) mz_ = fmin(mz_, fabs(lz[m]));
-    }
-    mn = mx_ * my_ * mz_;
-  }
-  constexpr int NZ = (D == 3) ? NP : 1;
-  if (!flip) {
-    const __amdgpu_buffer_rsrc_t rs = dir_rsrc<T>(a, own);
-    const int b0 = (int)base * (int)sizeof(T);
-#pragma unroll 1
-    for (int mz0 = 0; mz0 < NZ; mz0 += ZU) {
-#pragma unroll
-      for (int dz = 0; dz < ZU; dz++) {
-        const int mz = mz0 + dz;
-        if (NZ % ZU != 0 && mz >= NZ) break;
-        double accz = 0;
-#pragma unroll
-        for (int my = 0; my <= P; my++) {
-          double v[NP];
-          load_row<P, T>(rs, b0 + (int)sizeof(T) * (n0 * (my + n1 * mz)), v);
-          double row = lx[0] * v[0];
-#pragma unroll
-          for (int mx = 1; mx <= P; mx++) row += lx[mx] * v[mx];
-          accz += ly[my] * row;
-        }
-        acc += ((D == 3) ? lz[mz] : 1.0) * accz;
-      }
-    }
-    if (!(mn >= 1e-10)) acc = kept_sum<D, P, T>(rs, b0, n0, n1, lx, ly, lz);
-  } else if constexpr (D == 2) {
-#pragma unroll
-    for (int my = 0; my <= P; my++)
-#pragma unroll
-      for (int mx = 0; mx <= P; mx++) {
-        const double w = lx[mx] * ly[my];
-        if (!(fabs(w) < 1e-10)) acc += w * (double)src[base + mx + (int64_t)n0 * my];
-      }
+  bool cut = false;
+  int b0 = 0;
+  if (rec.c < 0) {
+    acc = (double)own[i];  // tracker life-time limit: identity row
   } else {
-#pragma unroll 1
-    for (int mz = 0; mz <= P; mz++)
+    const int64_t base = dep_weights<D, P, T>(a, dgl, rec, lx, ly, lz);
+    constexpr int NZ = (D == 3) ? NP : 1;
+    if (!flip) {
+      double mx_ = min_abs(lx[0], lx[1]), my_ = min_abs(ly[0], ly[1]), mz_ = (D == 3) ? min_abs(lz[0], lz[1]) : 1.0;
 #pragma unroll
-      for (int my = 0; my <= P; my++)
+      for (int m = 2; m <= P; m++) {
+        mx_ = min_abs(mx_, lx[m]);
+        my_ = min_abs(my_, ly[m]);
+        if constexpr (D == 3) mz_ = min_abs(mz_, lz[m]);
+      }
+      cut = !(mx_ * my_ * mz_ >= 1e-10);
+      b0 = (int)base * (int)sizeof(T);
+      if (!cut)  // (waves of x-face DoFs: every lane is cut in the directions along the face)
 #pragma unroll
-        for (int mx = 0; mx <= P; mx++) {
-          const double w = lx[mx] * ly[my] * lz[mz];
-          if (!(fabs(w) < 1e-10)) acc += w * (double)src[base + mx + (int64_t)n0 * (my + (int64_t)n1 * mz)];
+      for (int mz0 = 0; mz0 < NZ; mz0 += ZU) {
+#pragma unroll
+        for (int dz = 0; dz < ZU; dz++) {
+          const int mz = mz0 + dz;
+          if (NZ % ZU != 0 && mz >= NZ) break;
+          double accz = 0;
+#pragma unroll
+          for (int my = 0; my <= P; my++) {
+            double v[NP];
+            load_row<P, T>(rs, b0 + (int)sizeof(T) * (n0 * (my + n1 * mz)), v);
+            double row = fma(lx[0], v[0], lx[1] * v[1]);
+#pragma unroll
+            for (int mx = 2; mx <= P; mx++) row = fma(lx[mx], v[mx], row);
+            accz = fma(ly[my], row, accz);
+          }
+          acc = (D == 3) ? fma(lz[mz], accz, acc) : acc + accz;
         }
+        // ZU planes of rows in flight: reading further ahead would cost registers, and waves
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      const T* src = a.fin + (int64_t)opposite<Q>(al) * a.stride;
+#pragma unroll 1
+      for (int mz = 0; mz < NZ; mz++)
+#pragma unroll
+        for (int my = 0; my <= P; my++)
+#pragma unroll
+          for (int mx = 0; mx <= P; mx++) {
+            const double w = (D == 3) ? lx[mx] * ly[my] * lz[mz] : lx[mx] * ly[my];
+            if (!(fabs(w) < 1e-10)) acc = fma(w, (double)src[base + mx + (int64_t)n0 * (my + (int64_t)n1 * mz)], acc);
+          }
+    }
   }
+  if (__any(cut)) acc = kept_wave<D, P, T, R>(rs, cut, b0, n0, n1, lx, ly, lz, acc, sc);
   return (T)(acc + bias);
 }
 
@@ -374,54 +465,72 @@ __device__ __forceinline__ int64_t dof_of(const GeneralArgs<T>& a, int64_t g) {
   return (r0 + (h >> 1)) * nfe0 + ((h & 1) ? nfe0 - 1 : 0);
 }
 
-template <int D, int Q, int P, typename T, bool DEEP>
-__global__ __launch_bounds__((GeneralShape<D, Q, P, T, DEEP>::bs)) __attribute__((amdgpu_waves_per_eu(GeneralShape<D, Q, P, T, DEEP>::waves))) void k_sl_general(
+template <int D, int Q, int P, typename T, bool WIDE>
+__global__ __launch_bounds__((GeneralShape<D, Q, P, T, WIDE>::nt)) __attribute__((amdgpu_waves_per_eu(GeneralShape<D, Q, P, T, WIDE>::waves))) void k_sl_general(
     GeneralArgs<T> a, CollideArgs<T> ca, int write_macro) {
-  using S = GeneralShape<D, Q, P, T, DEEP>;
-  const int64_t g = xcd_block_index() * blockDim.x + threadIdx.x;
-  if (g >= a.n) return;
-  // the grouped order where it measured faster: the LDS forms at six waves (FP32) and four
-  // (FP64); the DEEP form and the FP64 D3Q27 register form keep the lattice order
-  const int64_t i = (S::lds && !DEEP) ? dof_of(a, g) : g;
-  int widx = -1;
-  unsigned wmask = 0;
-  if (a.wall_idx) {
-    widx = a.wall_idx[i];
-    if (widx >= 0) wmask = a.wall_flip[widx];
+  using S = GeneralShape<D, Q, P, T, WIDE>;
+  constexpr int G = S::G, W = S::W, bs = S::bs;
+  __shared__ __align__(16) T col[Q - 1][bs];
+  __shared__ double scr[S::R > 0 ? W * S::R * S::row_bytes / 8 : 1];
+  __shared__ int dofs[bs];
+  // FP32 records: differences of the GLL nodes, read with lane-dependent rows
+  __shared__ double dgl[sizeof(T) == 4 ? (P + 1) * (P + 1) : 1];
+  const int t = threadIdx.x;
+  if constexpr (sizeof(T) == 4)
+    if (t < (P + 1) * (P + 1)) dgl[t] = a.dgl[t / (P + 1)][t % (P + 1)];
+  if (t < bs) {
+    // threads beyond the mesh repeat its last DoF and store nothing
+    const int64_t g = xcd_block_index() * bs + t;
+    dofs[t] = (int)dof_of(a, g < a.n ? g : a.n - 1);
   }
-  T fs[Q];
-  if constexpr (S::lds) {
-    fs[0] = a.fin[i];
-    __shared__ T col[Q - 1][S::bs];
-    const int t = threadIdx.x;
-    if constexpr (S::prefetch) {
-      // the next direction's record is loaded before this direction's gathers, so its
-      // latency overlaps them (C3 FP64 370 -> 358 us per step; FP32 at 6 waves, at its
-      // 80-register cap, spilled more and lost 14%)
-      DepRec<D, T> rec = load_rec<D, T>(a, i);
+  __syncthreads();
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+  double* const sc = scr + (S::R > 0 ? w * S::R * S::row_bytes / 8 : 0);
+  // item k: direction 1 + k / G of group (k + k / G) mod G
+  struct Item {
+    int al, at;
+    int64_t i;
+    DepRec<D, T> rec;
+    int widx;
+  };
+  const auto fetch = [&](int k) {
+    Item it;
+    it.al = 1 + k / G;
+    it.at = ((k + k / G) % G) * 64 + lane;
+    it.i = dofs[it.at];
+    it.rec = load_rec<D, T>(a, (int64_t)(it.al - 1) * a.n + it.i);
+    it.widx = a.wall_idx ? a.wall_idx[it.i] : -1;
+    return it;
+  };
+  const auto stream = [&](const Item& it) {
+    const unsigned wmask = it.widx >= 0 ? a.wall_flip[it.widx] : 0u;
+    col[it.al - 1][it.at] = gen_direction<D, Q, P, T, S::zu, S::R>(a, dgl, sc, it.i, it.al, it.widx, wmask, it.rec);
+  };
+  constexpr int NI = G * (Q - 1);
+  if constexpr (S::prefetch) {
+    // the next item's record is loaded before this item's gathers, so its latency overlaps them
+    Item it = fetch(w < NI ? w : 0);
 #pragma unroll 1
-      for (int al = 1; al < Q; al++) {
-        DepRec<D, T> next = rec;
-        if (al + 1 < Q) next = load_rec<D, T>(a, (int64_t)al * a.n + i);
-        col[al - 1][t] = gen_direction<D, Q, P, T, S::zu>(a, i, al, widx, wmask, rec);
-        rec = next;
-      }
-    } else {
-#pragma unroll 1
-      for (int al = 1; al < Q; al++)
-        col[al - 1][t] =
-            gen_direction<D, Q, P, T, S::zu>(a, i, al, widx, wmask, load_rec<D, T>(a, (int64_t)(al - 1) * a.n + i));
+    for (int k = w; k < NI; k += W) {
+      Item next = it;
+      if (k + W < NI) next = fetch(k + W);
+      stream(it);
+      it = next;
     }
-    // keep the compiler from forwarding the stores into registers held across the loop
-    asm volatile("" ::: "memory");
-#pragma unroll
-    for (int al = 1; al < Q; al++) fs[al] = col[al - 1][t];
   } else {
-#pragma unroll
-    for (int al = 1; al < Q; al++)
-      fs[al] = gen_direction<D, Q, P, T, S::zu>(a, i, al, widx, wmask, load_rec<D, T>(a, (int64_t)(al - 1) * a.n + i));
-    fs[0] = a.fin[i];  // not held across the unrolled loop (FP64 D3Q27 p = 3: 181 -> 143 us)
+#pragma unroll 1
+    for (int k = w; k < NI; k += W) stream(fetch(k));
   }
+  __syncthreads();
+  if (w >= G) return;
+  // wave w collides group w
+  const int64_t g = xcd_block_index() * bs + t;
+  if (g >= a.n) return;
+  const int64_t i = dofs[t];
+  T fs[Q];
+  fs[0] = a.fin[i];
+#pragma unroll
+  for (int al = 1; al < Q; al++) fs[al] = col[al - 1][t];
   if (write_macro & STEP_STREAM_ONLY) {  // the SL stream with its wall values (CFDSolver::stream)
 #pragma unroll
     for (int q = 0; q < Q; q++) a.fout[(int64_t)q * a.stride + i] = fs[q];
@@ -430,32 +539,28 @@ __global__ __launch_bounds__((GeneralShape<D, Q, P, T, DEEP>::bs)) __attribute__
   bgk_collide_store_pairs<Q, T>(fs, ca, i, (write_macro & STEP_MACRO) != 0, a.fout, a.stride);
 }
 
-template <int D, int Q, int P, typename T, bool DEEP>
+template <int D, int Q, int P, typename T, bool WIDE>
 static int launch_general_shape(nat_ctx* ctx, const GeneralArgs<T>& a, const CollideArgs<T>& ca, int wm) {
-  constexpr int bs = GeneralShape<D, Q, P, T, DEEP>::bs;
-  hipLaunchKernelGGL((k_sl_general<D, Q, P, T, DEEP>), dim3((unsigned)((a.n + bs - 1) / bs)), dim3(bs), 0,
+  using S = GeneralShape<D, Q, P, T, WIDE>;
+  hipLaunchKernelGGL((k_sl_general<D, Q, P, T, WIDE>), dim3((unsigned)((a.n + S::bs - 1) / S::bs)), dim3(S::nt), 0,
                      ctx->stream, a, ca, wm);
   NAT_HIP(hipGetLastError());
   return 0;
 }
 
-// The DEEP form (FP32 3D only) when the autotuner chose it or, by default, when its grid fits
-// one round: 4 blocks of 256 DoFs per CU at 4 waves per SIMD.
+// The wide form when the autotuner or the caller chose it (FP32 3D) or, by default, up to 5/2
+// blocks per CU, where the other form leaves a SIMD with few waves (figures at GeneralShape; FP32
+// 460 blocks: equal; 887: 73 us against 74; FP64 516 blocks: 11.4 against 9.5; 920: 41 against 44).
 template <int D, int Q, int P, typename T>
-static bool deep_form(const nat_ctx* ctx, int64_t n) {
-  if constexpr (sizeof(T) == 4 && D == 3) {
-    constexpr int bs = GeneralShape<D, Q, P, T, true>::bs;
-    const int64_t blocks = (n + bs - 1) / bs;
-    return ctx->gen_pref >= 0 ? ctx->gen_pref == 1 : (ctx->n_cu > 0 && blocks <= 4 * (int64_t)ctx->n_cu);
-  } else {
-    return false;
-  }
+static bool wide_form(const nat_ctx* ctx, int64_t n) {
+  if (sizeof(T) == 4 && D == 3 && ctx->gen_pref >= 0) return ctx->gen_pref == 1;
+  constexpr int bs = GeneralShape<D, Q, P, T, true>::bs;
+  return 2 * ((n + bs - 1) / bs) <= 5 * (int64_t)ctx->n_cu;
 }
 
 template <int D, int Q, int P, typename T>
 static int launch_general(nat_ctx* ctx, const GeneralArgs<T>& a, const CollideArgs<T>& ca, int wm) {
-  if constexpr (sizeof(T) == 4 && D == 3)
-    if (deep_form<D, Q, P, T>(ctx, a.n)) return launch_general_shape<D, Q, P, T, true>(ctx, a, ca, wm);
+  if (wide_form<D, Q, P, T>(ctx, a.n)) return launch_general_shape<D, Q, P, T, true>(ctx, a, ca, wm);
   return launch_general_shape<D, Q, P, T, false>(ctx, a, ca, wm);
 }
 
@@ -592,8 +697,8 @@ int nat_launch_sl_general(nat_ctx* ctx, int write_macro) {
   return rc;
 }
 
-// Form of the general SL kernel picked by measurement. FP32 3D contexts have two (the
-// six-wave form and the DEEP form): each is timed for nsteps steps on the context's own mesh,
+// Form of the general SL kernel picked by measurement. FP32 3D contexts have two (eight
+// or sixteen waves per block): each is timed for nsteps steps on the context's own mesh,
 // writing the idle ping-pong buffer (populations, fields and time stay as they were), and the
 // faster is kept for this context and, process-wide, for later contexts of the same
 // instantiation and DoF count. Both forms run the same arithmetic in the same order, so
@@ -668,12 +773,15 @@ int nat_internal_autotune_general(nat_ctx* ctx, int nsteps, int* tile, double* b
       tile[2] = S::zu;
     };
     if (ctx->fp32) {
-      if (deep_form<D, Q, P, float>(ctx, ctx->n_dofs))
+      if (wide_form<D, Q, P, float>(ctx, ctx->n_dofs))
         put(GeneralShape<D, Q, P, float, true>{});
       else
         put(GeneralShape<D, Q, P, float, false>{});
     } else {
-      put(GeneralShape<D, Q, P, double, false>{});
+      if (wide_form<D, Q, P, double>(ctx, ctx->n_dofs))
+        put(GeneralShape<D, Q, P, double, true>{});
+      else
+        put(GeneralShape<D, Q, P, double, false>{});
     }
     return 0;
   });
