@@ -209,69 +209,136 @@ __device__ __forceinline__ void lag_all(const double (&x)[MAXP + 1], const doubl
   }
 }
 
+// A departure record: cell (-1: identity row) and unit coordinates.
+struct CompRec {
+  int c;
+  double xi0, xi1;
+};
+
+template <typename T>
+__device__ __forceinline__ CompRec comp_record(const CompArgs<T>& a, int al, int64_t i) {
+  const int64_t r = (int64_t)(al - 1) * a.n + i;
+  const double2 x = reinterpret_cast<const double2*>(a.xi)[r];
+  return {a.cell[r], x.x, x.y};
+}
+
+// Buffer resource from a direction's array on, for 32-bit byte offsets (uniform base). Opposite
+// directions are two arrays apart and an array is below 2 GiB (the records of a larger mesh do
+// not fit the device), so offsets into either stay below 2^32.
+template <typename T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t comp_rsrc(const T* p) {
+  const uint64_t pb = (uint64_t)p;
+  const uint32_t phi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(pb >> 32));
+  const uint32_t plo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)pb);
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(((uint64_t)phi << 32) | (uint64_t)plo), (short)0,
+                                           (int)0xffffffffu, 0x00020000);
+}
+
+// A row of P + 1 values in the fewest loads of 16, 12, 8 and 4 bytes.
+template <int P, typename T>
+__device__ __forceinline__ void comp_row(__amdgpu_buffer_rsrc_t r, int off, T (&v)[P + 1]) {
+  constexpr int W = (int)sizeof(T) / 4, ND = (P + 1) * W;
+  unsigned q[ND];
+  static_for<0, (ND + 3) / 4>([&](auto K) {
+    constexpr int k = 4 * decltype(K)::value, n = ND - k < 4 ? ND - k : 4;
+    if constexpr (n == 4) {
+      const auto x = __builtin_amdgcn_raw_buffer_load_b128(r, off + 4 * k, 0, 0);
+      static_for<0, 4>([&](auto J) { q[k + decltype(J)::value] = x[decltype(J)::value]; });
+    } else if constexpr (n == 3) {
+      const auto x = __builtin_amdgcn_raw_buffer_load_b96(r, off + 4 * k, 0, 0);
+      static_for<0, 3>([&](auto J) { q[k + decltype(J)::value] = x[decltype(J)::value]; });
+    } else if constexpr (n == 2) {
+      const auto x = __builtin_amdgcn_raw_buffer_load_b64(r, off + 4 * k, 0, 0);
+      static_for<0, 2>([&](auto J) { q[k + decltype(J)::value] = x[decltype(J)::value]; });
+    } else {
+      q[k] = __builtin_amdgcn_raw_buffer_load_b32(r, off + 4 * k, 0, 0);
+    }
+  });
+#pragma unroll
+  for (int m = 0; m <= P; m++) {
+    if constexpr (W == 1)
+      v[m] = __builtin_bit_cast(float, q[m]);
+    else
+      v[m] = __builtin_bit_cast(double, ((unsigned long)q[2 * m + 1] << 32) | q[2 * m]);
+  }
+}
+
+__device__ __forceinline__ double comp_min_abs(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
 // Streamed f and g of direction al at DoF i (al uniform across the wave), with the
-// FP32 shift added back. One set of FP64 weights serves f and g.
+// FP32 shift added back. One set of FP64 weights serves f and g. The stencil's rows are loaded
+// whole; where a product weight is under the cut-off (on the Cartesian meshes every lane of the
+// directions along an axis) the terms are dropped by selects, not by branches around their loads.
+// Lanes whose path was reflected at a wall read the opposite direction's array.
 template <int Q, int P, typename T>
 __device__ __forceinline__ void comp_stream_dir(const CompArgs<T>& a, const double* __restrict__ tab, int64_t i,
-                                                int al, int widx, unsigned wmask, double& fo, double& go) {
+                                                int al, int widx, unsigned wmask, const CompRec& rec, double& fo,
+                                                double& go) {
   const int n0 = a.nfe[0];
-  const int64_t r = (int64_t)(al - 1) * a.n + i;
-  const int sd = ((wmask >> al) & 1u) ? a.opp[al] : al;
-  const T* fsrc = a.fin + (int64_t)sd * a.stride;
-  const T* gsrc = a.gin + (int64_t)sd * a.stride;
+  const bool flip = (wmask >> al) & 1u;
   const double bias = widx >= 0 ? a.wall_bias[(int64_t)widx * Q + al] : 0.0;
-  const int c = a.cell[r];
+  const int c = rec.c;
   double af, ag;
   if (c < 0) {
     af = (double)a.fin[(int64_t)al * a.stride + i];
     ag = (double)a.gin[(int64_t)al * a.stride + i];
   } else {
     double lx[P + 1], ly[P + 1];
-    lag_all<P>(a.gll, a.inv_den, a.xi[2 * r + 0], lx);
-    lag_all<P>(a.gll, a.inv_den, a.xi[2 * r + 1], ly);
+    lag_all<P>(a.gll, a.inv_den, rec.xi0, lx);
+    lag_all<P>(a.gll, a.inv_den, rec.xi1, ly);
     const int cy = (int)a.divN0.div((uint32_t)c), cx = c - cy * a.N[0];
-    const int64_t base = (int64_t)cx * P + (int64_t)n0 * ((int64_t)cy * P);
+    const int base = cx * P + n0 * (cy * P);
     af = 0;
     ag = 0;
-    double mnx = fabs(lx[0]), mny = fabs(ly[0]);
+    // one resource over the direction and its opposite: a reflected lane adds their distance
+    const int lo = al < a.opp[al] ? al : a.opp[al];
+    const __amdgpu_buffer_rsrc_t rf = comp_rsrc(a.fin + (int64_t)lo * a.stride),
+                                 rg = comp_rsrc(a.gin + (int64_t)lo * a.stride);
+    const unsigned src = (unsigned)((flip ? a.opp[al] : al) - lo) * (unsigned)(a.stride * (int64_t)sizeof(T));
+    double mnx = comp_min_abs(lx[0], lx[1]), mny = comp_min_abs(ly[0], ly[1]);
 #pragma unroll
-    for (int m = 1; m <= P; m++) {
-      mnx = fmin(mnx, fabs(lx[m]));
-      mny = fmin(mny, fabs(ly[m]));
+    for (int m = 2; m <= P; m++) {
+      mnx = comp_min_abs(mnx, lx[m]);
+      mny = comp_min_abs(mny, ly[m]);
     }
-    if (mnx * mny >= 1e-10) {
-      // no product weight reaches the cut-off: every term is taken, with the loads of
-      // the whole stencil issued together (same terms in the same order)
-      double vf[P + 1][P + 1], vg[P + 1][P + 1];
+    const bool cut = __any(!(mnx * mny >= 1e-10));
+    constexpr int R = P <= 3 ? P + 1 : 2;  // rows in flight at a time (p = 4, all 5: 208 VGPRs, 96^2 84 us, not 67)
+    static_for<0, (P + R) / R>([&](auto G) {
+      constexpr int y0 = decltype(G)::value * R, ny = P + 1 - y0 < R ? P + 1 - y0 : R;
+      T vf[ny][P + 1], vg[ny][P + 1];
 #pragma unroll
-      for (int my = 0; my <= P; my++)
+      for (int y = 0; y < ny; y++) {
+        const int off = (int)(src + (unsigned)(base + n0 * (y0 + y)) * (unsigned)sizeof(T));
+        comp_row<P, T>(rf, off, vf[y]);
+        comp_row<P, T>(rg, off, vg[y]);
+      }
+      if (!cut) {
+        // no product weight reaches the cut-off: every term is taken
 #pragma unroll
-        for (int mx = 0; mx <= P; mx++) {
-          const int64_t k = base + mx + (int64_t)n0 * my;
-          vf[my][mx] = (double)fsrc[k];
-          vg[my][mx] = (double)gsrc[k];
-        }
+        for (int y = 0; y < ny; y++)
 #pragma unroll
-      for (int my = 0; my <= P; my++)
-#pragma unroll
-        for (int mx = 0; mx <= P; mx++) {
-          const double w = lx[mx] * ly[my];
-          af += w * vf[my][mx];
-          ag += w * vg[my][mx];
-        }
-    } else {
-#pragma unroll
-      for (int my = 0; my <= P; my++)
-#pragma unroll
-        for (int mx = 0; mx <= P; mx++) {
-          const double w = lx[mx] * ly[my];
-          if (!(fabs(w) < 1e-10)) {
-            const int64_t k = base + mx + (int64_t)n0 * my;
-            af += w * (double)fsrc[k];
-            ag += w * (double)gsrc[k];
+          for (int mx = 0; mx <= P; mx++) {
+            const double w = lx[mx] * ly[y0 + y];
+            af = fma(w, (double)vf[y][mx], af);
+            ag = fma(w, (double)vg[y][mx], ag);
           }
-        }
-    }
+      } else {
+#pragma unroll
+        for (int y = 0; y < ny; y++)
+#pragma unroll
+          for (int mx = 0; mx <= P; mx++) {
+            const double w = lx[mx] * ly[y0 + y];
+            const bool keep = !(fabs(w) < 1e-10);
+            const double sf = fma(w, (double)vf[y][mx], af), sg = fma(w, (double)vg[y][mx], ag);
+            af = keep ? sf : af;
+            ag = keep ? sg : ag;
+          }
+      }
+    });
   }
   af = af + bias;
   fo = af + tab[al * CTAB + CT_W] * a.rho0;
@@ -279,33 +346,38 @@ __device__ __forceinline__ void comp_stream_dir(const CompArgs<T>& a, const doub
 }
 
 // Fused SL stream of f and g + compressible collision. The work of a block is spread
-// over its waves: 64 DoFs per block, CW waves each streaming every CW-th direction of
-// those DoFs (one thread per DoF would give a 66k-DoF grid only four waves per CU to hide
-// its gather latency). The streamed values meet in LDS. The collision is spread the
-// same way: each wave sums the moments over its own directions, the partial sums meet in
-// LDS and are added in wave order (so a run is reproducible), every wave forms the node
-// state from them and relaxes its own directions. Without a Prandtl number the
-// equilibrium of a direction serves both its Knudsen term and its relaxation; with one
-// (PR) the third moments must be complete first, through one more LDS reduction.
-// Waves per block: 8, or 4 with a Prandtl number, whose 11-value reduction buffer would
-// otherwise leave room for one block per CU (C4 with Pr = 0.71: 0.97 -> 1.60 GLUPS FP32;
-// 8 waves measured best without it).
+// over its waves: 64 DoFs per block, CW waves, wave w streaming and relaxing the directions
+// w, w + CW, ... of those DoFs and holding their values in registers throughout (one thread per
+// DoF would give a 66k-DoF grid only four waves per CU to hide its gather latency). The moments
+// are summed over classes of directions, q modulo CL; the partial sums meet in LDS and are added
+// in class order, so neither a repeated run nor another CW changes a bit. Every wave forms the
+// node state from them and relaxes its own directions. Without a Prandtl number the equilibrium
+// of a direction serves both its Knudsen term and its relaxation; with one (PR) the third moments
+// must be complete first, through one more LDS reduction. Its 11-value reduction buffer allows 4
+// classes only (8 would leave room for one block per CU; 128^2 p=2 with Pr = 0.71: 0.97 -> 1.60
+// GLUPS FP32).
+// Bound by the latency of a wave's serial chain (record, rows, sums; a step moves about 57 MB at
+// 128^2 p=2 FP32, 9 us at the cache's rate), so the record of the next direction is loaded ahead
+// and the rows come in whole-row loads that no branch splits. Against single loads with the cut
+// terms behind branches and the values kept in LDS, us per step (FP32, FP64; walls in y):
+// p=2 16^2 11.3 -> 9.6, 12.1 -> 9.5; p=2 128^2 29.2 -> 26.0, 33.0 -> 26.6; p=3 64^2 32.2 -> 18.4,
+// 34.9 -> 22.5; p=2 256^2 80.2 -> 61.5, 121 -> 90; Pr 0.71 128^2 40.5 -> 34.2, 44.0 -> 35.7. Also
+// fetching the next direction's rows ahead (156 VGPRs) is faster on 128^2 FP32 without walls
+// (25.1 -> 22.7) and slower elsewhere.
 template <bool PR>
-constexpr int comp_waves() {
+constexpr int comp_classes() {
   return PR ? 4 : 8;
 }
 // ST = false: no streaming, each DoF's own populations are collided in place (the
 // initial collision of CFDSolver::run; fin and fout may be the same arrays, since every
-// value of the block is read into LDS before the barrier and only this block touches
-// its 64 DoFs).
-template <int Q, int P, typename T, bool PR, bool ST = true>
-__global__ __launch_bounds__(comp_waves<PR>() * 64) void k_sl_comp_wide(CompArgs<T> a,
-                                                                        const double* __restrict__ tab,
-                                                                        int write_macro) {
-  constexpr int CW = comp_waves<PR>();
+// value is read before it is written and only this block touches its 64 DoFs).
+template <int Q, int P, typename T, bool PR, bool ST = true, int CW = comp_classes<PR>()>
+__global__ __launch_bounds__(CW * 64) void k_sl_comp_wide(CompArgs<T> a, const double* __restrict__ tab,
+                                                          int write_macro) {
+  constexpr int CL = comp_classes<PR>(), NC = CL / CW;  // a wave holds NC classes
+  constexpr int NK = (Q + CW - 1) / CW;  // directions of a wave, the last of them of the first waves only
   constexpr int NV = PR ? 11 : 5;  // kn, Q (8), F (2); moments: rho, j (3) + tf, tg (2)
-  __shared__ double sf[Q][64], sg[Q][64];
-  __shared__ double red[CW][NV][64];
+  __shared__ double red[CL][NV][64];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int64_t i = (int64_t)blockIdx.x * 64 + lane;
@@ -318,70 +390,76 @@ __global__ __launch_bounds__(comp_waves<PR>() * 64) void k_sl_comp_wide(CompArgs
   }
   // stream only (uniform over the grid): each wave stores the directions it streamed
   const bool so = ST && a.stream_only;
+  double fv[NK], gv[NK];
+  // calls f(k, q) for the wave's k-th direction q
+  const auto each = [&](auto&& f) {
+    static_for<0, NK>([&](auto K) {
+      constexpr int k = decltype(K)::value;
+      const int q = w + k * CW;
+      if ((k + 1) * CW <= Q || q < Q) f(K, q);  // uniform
+    });
+  };
   if (live) {
-    if (w == 0) {
-      if (so) {
-        a.fout[i] = a.fin[i];
-        a.gout[i] = a.gin[i];
+    CompRec next{};
+    if constexpr (ST) next = comp_record<T>(a, w > 0 ? w : CW, i);  // (direction 0 has no record)
+    each([&](auto K, int q) {
+      constexpr int k = decltype(K)::value;
+      if (ST && q > 0) {
+        const CompRec rec = next;  // the next direction's record is loaded ahead of this one's stencil
+        if (q + CW < Q) next = comp_record<T>(a, q + CW, i);
+        comp_stream_dir<Q, P, T>(a, tab, i, q, widx, wmask, rec, fv[k], gv[k]);
+        if (so) {
+          a.fout[(int64_t)q * a.stride + i] = (T)(fv[k] - tab[q * CTAB + CT_W] * a.rho0);
+          a.gout[(int64_t)q * a.stride + i] = (T)(gv[k] - tab[q * CTAB + CT_W] * a.gshift);
+        }
       } else {
-        sf[0][lane] = (double)a.fin[i] + tab[CT_W] * a.rho0;
-        sg[0][lane] = (double)a.gin[i] + tab[CT_W] * a.gshift;
+        const T f = a.fin[(int64_t)q * a.stride + i], g = a.gin[(int64_t)q * a.stride + i];
+        if (so) {
+          a.fout[(int64_t)q * a.stride + i] = f;
+          a.gout[(int64_t)q * a.stride + i] = g;
+        }
+        fv[k] = (double)f + tab[q * CTAB + CT_W] * a.rho0;
+        gv[k] = (double)g + tab[q * CTAB + CT_W] * a.gshift;
       }
-    }
-    for (int al = 1 + w; al < Q; al += CW) {
-      double fo, go;
-      if constexpr (ST) {
-        comp_stream_dir<Q, P, T>(a, tab, i, al, widx, wmask, fo, go);
-      } else {
-        fo = (double)a.fin[(int64_t)al * a.stride + i] + tab[al * CTAB + CT_W] * a.rho0;
-        go = (double)a.gin[(int64_t)al * a.stride + i] + tab[al * CTAB + CT_W] * a.gshift;
-      }
-      if (so) {
-        a.fout[(int64_t)al * a.stride + i] = (T)(fo - tab[al * CTAB + CT_W] * a.rho0);
-        a.gout[(int64_t)al * a.stride + i] = (T)(go - tab[al * CTAB + CT_W] * a.gshift);
-      } else {
-        sf[al][lane] = fo;
-        sg[al][lane] = go;
-      }
-    }
+    });
   }
   if (so) return;
-  __syncthreads();
-  const auto fl = [&](int q) { return sf[q][lane]; };
-  const auto gl = [&](int q) { return sg[q][lane]; };
-  // moments: each wave sums its own directions; partial sums meet in LDS, added in wave order
-  double m0 = 0, m1 = 0, m2 = 0;
+  // moments: each wave sums its own classes; partial sums meet in LDS, added in class order
+  double m[NC][3] = {};
   if (live)
-    for (int q = w; q < Q; q += CW) {
-      const double f = fl(q);
-      m0 += f;
-      m1 += tab[q * CTAB + CT_E0] * f;
-      m2 += tab[q * CTAB + CT_E1] * f;
-    }
-  red[w][0][lane] = m0;
-  red[w][1][lane] = m1;
-  red[w][2][lane] = m2;
+    each([&](auto K, int q) {
+      constexpr int k = decltype(K)::value, c = k % NC;
+      m[c][0] += fv[k];
+      m[c][1] += tab[q * CTAB + CT_E0] * fv[k];
+      m[c][2] += tab[q * CTAB + CT_E1] * fv[k];
+    });
+#pragma unroll
+  for (int c = 0; c < NC; c++)
+#pragma unroll
+    for (int d = 0; d < 3; d++) red[w + c * CW][d][lane] = m[c][d];
   __syncthreads();
   double rho = red[0][0][lane], j0 = red[0][1][lane], j1 = red[0][2][lane];
-  for (int v = 1; v < CW; v++) {
+  for (int v = 1; v < CL; v++) {
     rho += red[v][0][lane];
     j0 += red[v][1][lane];
     j1 += red[v][2][lane];
   }
   const double u0 = j0 * (1.0 / rho), u1 = j1 * (1.0 / rho);
-  double tf = 0, tg = 0;
+  double mt[NC][2] = {};
   if (live)
-    for (int q = w; q < Q; q += CW) {
+    each([&](auto K, int q) {
+      constexpr int k = decltype(K)::value, c = k % NC;
       const double d0 = tab[q * CTAB + CT_E0] - u0, d1 = tab[q * CTAB + CT_E1] - u1;
-      tf += (d0 * d0 + d1 * d1) * fl(q);
-      tg += gl(q);
-    }
-  red[w][3][lane] = tf;
-  red[w][4][lane] = tg;
+      mt[c][0] += (d0 * d0 + d1 * d1) * fv[k];
+      mt[c][1] += gv[k];
+    });
+#pragma unroll
+  for (int c = 0; c < NC; c++)
+#pragma unroll
+    for (int d = 0; d < 2; d++) red[w + c * CW][3 + d][lane] = mt[c][d];
   __syncthreads();
-  tf = red[0][3][lane];
-  tg = red[0][4][lane];
-  for (int v = 1; v < CW; v++) {
+  double tf = red[0][3][lane], tg = red[0][4][lane];
+  for (int v = 1; v < CL; v++) {
     tf += red[v][3][lane];
     tg += red[v][4][lane];
   }
@@ -394,8 +472,11 @@ __global__ __launch_bounds__(comp_waves<PR>() * 64) void k_sl_comp_wide(CompArgs
   };
   CompNeq s;
   if constexpr (PR) {
+    static_assert(NC == 1, "one class per wave");
     if (live)
-      for (int q = w; q < Q; q += CW) comp_neq_add<true, T>(s, nd, a, tab + q * CTAB, fl(q), gl(q));
+      each([&](auto K, int q) {
+        comp_neq_add<true, T>(s, nd, a, tab + q * CTAB, fv[decltype(K)::value], gv[decltype(K)::value]);
+      });
     __syncthreads();  // every wave has read the moment sums
     red[w][0][lane] = s.kn;
 #pragma unroll
@@ -409,7 +490,7 @@ __global__ __launch_bounds__(comp_waves<PR>() * 64) void k_sl_comp_wide(CompArgs
     for (int k = 0; k < 8; k++) t.Qt[k >> 2][(k >> 1) & 1][k & 1] = red[0][1 + k][lane];
     t.Fg[0] = red[0][9][lane];
     t.Fg[1] = red[0][10][lane];
-    for (int v = 1; v < CW; v++) {
+    for (int v = 1; v < CL; v++) {
       t.kn += red[v][0][lane];
 #pragma unroll
       for (int k = 0; k < 8; k++) t.Qt[k >> 2][(k >> 1) & 1][k & 1] += red[v][1 + k][lane];
@@ -417,27 +498,30 @@ __global__ __launch_bounds__(comp_waves<PR>() * 64) void k_sl_comp_wide(CompArgs
       t.Fg[1] += red[v][10][lane];
     }
     if (live)
-      for (int q = w; q < Q; q += CW) {
+      each([&](auto K, int q) {
         const double* tq = tab + q * CTAB;
         double fn, gn;
-        comp_relax<true, T>(nd, t, a, tq, nd.qn.feq(tq), fl(q), gl(q), fn, gn);
+        comp_relax<true, T>(nd, t, a, tq, nd.qn.feq(tq), fv[decltype(K)::value], gv[decltype(K)::value], fn, gn);
         store(q, fn, gn);
-      }
+      });
     s.kn = t.kn;
   } else {
+    CompNeq sc[NC];
     if (live)
-      for (int q = w; q < Q; q += CW) {
+      each([&](auto K, int q) {
+        constexpr int k = decltype(K)::value;
         const double* tq = tab + q * CTAB;
-        const double fe = comp_neq_add<false, T>(s, nd, a, tq, fl(q), gl(q));
+        const double fe = comp_neq_add<false, T>(sc[k % NC], nd, a, tq, fv[k], gv[k]);
         double fn, gn;
-        comp_relax<false, T>(nd, s, a, tq, fe, fl(q), gl(q), fn, gn);
+        comp_relax<false, T>(nd, sc[k % NC], a, tq, fe, fv[k], gv[k], fn, gn);
         store(q, fn, gn);
-      }
+      });
     if (write_macro) {  // uniform over the block
-      red[w][0][lane] = s.kn;
+#pragma unroll
+      for (int c = 0; c < NC; c++) red[w + c * CW][0][lane] = sc[c].kn;
       __syncthreads();
       s.kn = red[0][0][lane];
-      for (int v = 1; v < CW; v++) s.kn += red[v][0][lane];
+      for (int v = 1; v < CL; v++) s.kn += red[v][0][lane];
     }
   }
   if (write_macro && w == 0 && live) comp_write_macro<T>(a, nd, s.kn, Q, i);
@@ -501,6 +585,19 @@ static void fill_comp(nat_ctx* ctx, CompArgs<T>& a, int src, int dst) {
   a.stream_only = 0;
 }
 
+// Waves per block: 8 spread a DoF's directions over the CU while there is about a block for each
+// of the 256 CUs, 4 need fewer blocks' worth of waves at the barriers when there are more. FP32
+// (but for p = 3, whose registers leave one block of 8 waves per CU) gains from 8 a little longer.
+// us per step with 8 / 4 waves, walls in y, FP32 and FP64:
+//   p=2  66 blocks (32^2)   7.7/ 9.8   8.5/10.4      p=2 329 blocks (72^2)  11.4/11.8  14.3/13.4
+//   p=2 261 blocks (64^2)  11.3/11.5  14.1/13.2      p=2 512 blocks (90^2)  13.4/13.0  16.3/15.6
+//   p=3 263 blocks (43^2)  20.0/13.8  15.9/15.2      p=4 407 blocks (40^2)  16.9/17.9  21.0/20.6
+//   p=3 582 blocks (64^2)  24.2/18.4  22.8/22.5      p=2 1030 blocks (128^2) 27.1/26.1 31.0/26.2
+template <typename T>
+constexpr unsigned comp_blocks8(int p) {
+  return sizeof(T) == 4 && p != 3 ? 410 : 256;
+}
+
 template <typename T>
 static int step_comp(nat_ctx* ctx, int mode) {
   CompArgs<T> a;
@@ -510,25 +607,36 @@ static int step_comp(nat_ctx* ctx, int mode) {
   const int write_macro = (mode & STEP_MACRO) ? 1 : 0;
   const unsigned grid = (unsigned)((a.n + 63) / 64);
   const double* tab = ctx->comp_tab;
-  const dim3 blk(comp_waves<true>() * 64), blk0(comp_waves<false>() * 64);
-#define NAT_CW(PP)                                                                                              \
-  case PP:                                                                                                     \
-    if (a.prandtl_set)                                                                                         \
-      hipLaunchKernelGGL((k_sl_comp_wide<25, PP, T, true>), dim3(grid), blk, 0, ctx->stream, a, tab, write_macro); \
-    else                                                                                                       \
-      hipLaunchKernelGGL((k_sl_comp_wide<25, PP, T, false>), dim3(grid), blk0, 0, ctx->stream, a, tab,           \
-                         write_macro);                                                                         \
-    break;
+  const auto launch = [&](auto PP, auto PR, auto CW) {
+    hipLaunchKernelGGL((k_sl_comp_wide<25, decltype(PP)::value, T, decltype(PR)::value, true, decltype(CW)::value>),
+                       dim3(grid), dim3(decltype(CW)::value * 64), 0, ctx->stream, a, tab, write_macro);
+  };
+  const auto pick = [&](auto PP) {
+    using std::integral_constant;
+    if (a.prandtl_set)
+      launch(PP, std::true_type{}, integral_constant<int, 4>{});
+    else if (grid <= comp_blocks8<T>(decltype(PP)::value))
+      launch(PP, std::false_type{}, integral_constant<int, 8>{});
+    else
+      launch(PP, std::false_type{}, integral_constant<int, 4>{});
+  };
   switch (ctx->p) {
-    NAT_CW(1)
-    NAT_CW(2)
-    NAT_CW(3)
-    NAT_CW(4)
+    case 1:
+      pick(std::integral_constant<int, 1>{});
+      break;
+    case 2:
+      pick(std::integral_constant<int, 2>{});
+      break;
+    case 3:
+      pick(std::integral_constant<int, 3>{});
+      break;
+    case 4:
+      pick(std::integral_constant<int, 4>{});
+      break;
     default:
       ctx->err = "compressible SL kernel instantiated for p <= 4";
       return NAT_ERR_UNSUPPORTED;
   }
-#undef NAT_CW
   NAT_HIP(hipGetLastError());
   ctx->cur = dst;
   return 0;
@@ -541,10 +649,10 @@ static int collide_comp(nat_ctx* ctx) {
   const unsigned grid = (unsigned)((a.n + 63) / 64);
   const double* tab = ctx->comp_tab;
   if (a.prandtl_set)
-    hipLaunchKernelGGL((k_sl_comp_wide<25, 1, T, true, false>), dim3(grid), dim3(comp_waves<true>() * 64), 0,
+    hipLaunchKernelGGL((k_sl_comp_wide<25, 1, T, true, false>), dim3(grid), dim3(comp_classes<true>() * 64), 0,
                        ctx->stream, a, tab, 1);
   else
-    hipLaunchKernelGGL((k_sl_comp_wide<25, 1, T, false, false>), dim3(grid), dim3(comp_waves<false>() * 64), 0,
+    hipLaunchKernelGGL((k_sl_comp_wide<25, 1, T, false, false>), dim3(grid), dim3(comp_classes<false>() * 64), 0,
                        ctx->stream, a, tab, 1);
   NAT_HIP(hipGetLastError());
   return 0;
