@@ -36,8 +36,7 @@
 // FP32 storage keeps f~ = f - w rho0 in FP32. L annihilates constants for the
 // upwind flux; for the central flux L(w rho0) = w rho0 sum_a s_a G_a / w_a(i) is
 // added back explicitly. All arithmetic is FP64.
-#include "nat_collide.hpp"
-#include "nat_geom.hpp"
+#include "nat_sedg.hpp"
 
 namespace nat {
 
@@ -48,39 +47,9 @@ static const double kRkB[5] = {1432997174477.0 / 9575080441755.0, 5161836677717.
                                1720146321549.0 / 2090206949498.0, 3134564353537.0 / 4481467310338.0,
                                2277821191437.0 / 14882151754819.0};
 
-template <typename T>
-struct SedgArgs {
-  const T* fin;
-  T* fout;
-  T* df;
-  int64_t stride;
-  int64_t ncell;
-  MeshDev m;
-  double scaling;
-  double dt;
-  double a, b;       // RK5 coefficients of this stage
-  double binv;       // 1 / b (the division of df /= b is a multiplication by 1/b)
-  double rho0;       // FP32 shift (0 for FP64)
-  int first;         // first stage: df not read
-  int store_df;      // 0 on the last stage (df is dead afterwards)
-  int central;       // central flux
-  double gll[MAXP + 1];
-  double inv_gw[MAXP + 1];           // 1 / GLL weight
-  double dl[MAXP + 1][MAXP + 1];     // dl[i][j] = phi_j'(x_i)
-};
-
-template <int D, int P>
-struct SedgShape {
-  static constexpr int NP = P + 1;
-  static constexpr int NL = (D == 3) ? NP * NP * NP : NP * NP;
-  // cells per block: ~256 threads; a 64-node cell (3D, p = 3) runs alone as one wave, whose
-  // per-direction barrier then waits for no other wave (C3 SEDG +4% FP32, +1% FP64)
-  static constexpr int CPB = (NL == 64) ? 1 : ((256 / NL) > 0 ? 256 / NL : 1);
-  static constexpr int NT = CPB * NL;
-};
-
-__device__ __forceinline__ void sedg_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
+// General stage kernel, one direction at a time: the central flux, and the upwind flux of meshes
+// whose arrays exceed the offsets of the pairwise kernel.
+//
 // WALLS: the mesh has a non-periodic axis (its own instantiation: the wall terms cost
 // registers that the periodic kernels keep for occupancy)
 template <int D, int Q, int P, typename T, bool COL, bool WALLS>
@@ -174,9 +143,9 @@ __global__ __launch_bounds__((SedgShape<D, P>::NT)) void k_sedg_stage(SedgArgs<T
     }
     // Face neighbours this direction reads. With FP64 storage they are loaded before the
     // barrier, so that their latency overlaps the LDS exchange and the volume term
-    // (C3 SEDG FP64 0.88 -> 1.14 GLUPS). With FP32 storage they are loaded right after
+    // (24^3 p=3 D3Q19 FP64 0.88 -> 1.14 GLUPS). With FP32 storage they are loaded right after
     // the barrier, so that the volume term covers their latency: the stage then holds
-    // 110 registers (4 waves per SIMD) and C3 FP32 takes 621 us per step, against 707
+    // 110 registers (4 waves per SIMD) and the FP32 step takes 621 us, against 707
     // with the loads after the volume term (131 registers, 3 waves) and 758 before the
     // barrier.
     constexpr bool early = sizeof(T) == 8;
@@ -270,6 +239,10 @@ static int launch_stage(nat_ctx* ctx, const SedgArgs<T>& s, const CollideArgs<T>
 template <typename T>
 static int dispatch_stage(nat_ctx* ctx, const SedgArgs<T>& s, const CollideArgs<T>& ca, int collide, int wm) {
   const int Q = ctx->Q, P = ctx->p;
+  if (!s.central && nat_sedg_pair_stage<T>(ctx, s, ca, collide, wm)) {
+    NAT_HIP(hipGetLastError());
+    return 0;
+  }
 #define NAT_SE(DD, QQ, PP) \
   if (Q == QQ && P == PP) return launch_stage<DD, QQ, PP, T>(ctx, s, ca, collide, wm);
   NAT_SE(2, 9, 1)
