@@ -35,59 +35,80 @@ __device__ __forceinline__ const double* cell_vertex(const MeshDev& m, const int
   return vtx(m, c[0] + (v & 1), c[1] + ((v >> 1) & 1), D == 3 ? c[2] + ((v >> 2) & 1) : 0);
 }
 
+// The cell a walk stands in and the address of its first vertex.
 template <int D>
-__device__ void map_fwd(const MeshDev& m, const int c[3], const double xi[3], double x[3]) {
-  const int nv = D == 3 ? 8 : 4;
+struct Cell {
+  static constexpr int NV = D == 3 ? 8 : 4;
+  int c[3];
+  const double* p;
+  int s1, s2;
+  __device__ __forceinline__ void load(const MeshDev& m) {
+    p = cell_vertex<D>(m, c, 0);
+    s1 = 3 * (m.N[0] + 1);
+    s2 = s1 * (m.N[1] + 1);
+  }
+  __device__ __forceinline__ double X(int v, int d) const {
+    return p[(v & 1) * 3 + ((v >> 1) & 1) * s1 + ((v >> 2) & 1) * s2 + d];
+  }
+};
+template <int D>
+__device__ __forceinline__ void map_fwd(const MeshDev& m, const Cell<D>& C, const double xi[3], double x[3]) {
+  constexpr int nv = Cell<D>::NV;
   if (m.cartesian) {
-    const double* a = cell_vertex<D>(m, c, 0);
-    const double* b = cell_vertex<D>(m, c, nv - 1);
-    for (int d = 0; d < 3; d++) x[d] = d < D ? a[d] + xi[d] * (b[d] - a[d]) : 0.0;
+#pragma unroll
+    for (int d = 0; d < D; d++) x[d] = C.X(0, d) + xi[d] * (C.X(nv - 1, d) - C.X(0, d));
+    if (D == 2) x[2] = 0.0;
     return;
   }
   x[0] = x[1] = x[2] = 0;
+#pragma unroll
   for (int v = 0; v < nv; v++) {
     double Nv = 1;
+#pragma unroll
     for (int a = 0; a < D; a++) Nv *= ((v >> a) & 1) ? xi[a] : (1 - xi[a]);
-    const double* X = cell_vertex<D>(m, c, v);
-    for (int d = 0; d < D; d++) x[d] += Nv * X[d];
+#pragma unroll
+    for (int d = 0; d < D; d++) x[d] += Nv * C.X(v, d);
   }
 }
 
 template <int D>
-__device__ void jac(const MeshDev& m, const int c[3], const double xi[3], double J[3][3]) {
+__device__ __forceinline__ void jac(const Cell<D>& C, const double xi[3], double J[3][3]) {
+#pragma unroll
   for (int a = 0; a < 3; a++)
+#pragma unroll
     for (int b = 0; b < 3; b++) J[a][b] = (a == b && a >= D) ? 1.0 : 0.0;
-  const int nv = D == 3 ? 8 : 4;
-  for (int v = 0; v < nv; v++) {
-    const double* X = cell_vertex<D>(m, c, v);
+#pragma unroll
+  for (int v = 0; v < Cell<D>::NV; v++) {
+#pragma unroll
     for (int b = 0; b < D; b++) {
       double dN = 1;
+#pragma unroll
       for (int a = 0; a < D; a++) {
         const int bit = (v >> a) & 1;
         dN *= (a == b) ? (bit ? 1.0 : -1.0) : (bit ? xi[a] : 1 - xi[a]);
       }
-      for (int d = 0; d < D; d++) J[d][b] += dN * X[d];
+#pragma unroll
+      for (int d = 0; d < D; d++) J[d][b] += dN * C.X(v, d);
     }
   }
 }
 
 // inverse map; false when the Newton iteration of the multilinear map fails
 template <int D>
-__device__ bool map_inv(const MeshDev& m, const int c[3], const double x[3], double xi[3]) {
-  const int nv = D == 3 ? 8 : 4;
+__device__ bool map_inv(const MeshDev& m, const Cell<D>& C, const double x[3], double xi[3]) {
   if (m.cartesian) {
-    const double* a = cell_vertex<D>(m, c, 0);
-    const double* b = cell_vertex<D>(m, c, nv - 1);
-    for (int d = 0; d < 3; d++) xi[d] = d < D ? (x[d] - a[d]) / (b[d] - a[d]) : 0.0;
+#pragma unroll
+    for (int d = 0; d < D; d++) xi[d] = (x[d] - C.X(0, d)) / (C.X(Cell<D>::NV - 1, d) - C.X(0, d));
+    if (D == 2) xi[2] = 0.0;
     return true;
   }
   for (int d = 0; d < 3; d++) xi[d] = d < D ? 0.5 : 0.0;
   double prev = 1e300;
   for (int it = 0; it < 100; it++) {
     double y[3], J[3][3], r[3], s[3];
-    map_fwd<D>(m, c, xi, y);
+    map_fwd<D>(m, C, xi, y);
     for (int d = 0; d < 3; d++) r[d] = d < D ? y[d] - x[d] : 0.0;
-    jac<D>(m, c, xi, J);
+    jac<D>(C, xi, J);
     if (D == 2) {
       const double det = J[0][0] * J[1][1] - J[0][1] * J[1][0];
       if (det == 0) return false;
@@ -190,10 +211,13 @@ __device__ int crossed_without_mapping(const MeshDev& m, const int c[3], const d
   return imin;
 }
 
+// Face through which the path pin -> pout leaves the cell (-1: pout is inside) and the crossing
+// point. pi: unit coordinates of pin, or !pi_ok where the inverse map fails; po: those of pout.
 template <int D>
-__device__ int crossed_first(const MeshDev& m, const int c[3], const double pin[3], const double pout[3], double pb[3]) {
-  double pi[3], po[3];
-  if (!map_inv<D>(m, c, pin, pi) || !map_inv<D>(m, c, pout, po)) return crossed_without_mapping<D>(m, c, pin, pout, pb);
+__device__ __forceinline__ int crossed_first(const MeshDev& m, const Cell<D>& C, const double pin[3],
+                                             const double pout[3], bool pi_ok, double pi[3], bool po_ok, double po[3],
+                                             double pb[3]) {
+  if (!pi_ok || !po_ok) return crossed_without_mapping<D>(m, C.c, pin, pout, pb);
   for (int i = 0; i < D; i++) {
     clamp01(pi[i]);
     clamp01(po[i]);
@@ -219,33 +243,40 @@ __device__ int crossed_first(const MeshDev& m, const int c[3], const double pin[
     h[i] = pi[i] + (po[i] - pi[i]) * lambda;
     clamp01(h[i]);
   }
-  map_fwd<D>(m, c, h, pb);
+  map_fwd<D>(m, C, h, pb);
   return face;
 }
 
-// Walk from the owning cell to the cell holding x - dt c. Returns the cell index,
-// -1 when the life-time limit is hit (identity row), -3 when the final unit point
-// is outside its cell. At a wall face the path turns into the opposite direction
-// at the hit point and continues for the remaining distance in the same cell;
+// Walk from the owning cell (C, where x has the unit coordinates p0) to the cell holding
+// x - dt c. Returns the cell index, -1 when the life-time limit is hit (identity row), -3 when
+// the final unit point is outside its cell. At a wall face the path turns into the opposite
+// direction at the hit point and continues for the remaining distance in the same cell;
 // *nhit counts the wall hits (an odd count reads the opposite direction) and *bias
 // accumulates 2 w (e . u_wall) / cs2 (rho = 1, destination direction e) per hit.
 template <int D>
-__device__ int locate(const MeshDev& m, int owner, const double x[3], const double disp[3], const double e[3],
-                      double w, double cs2, double xi[3], int* nhit, double* bias) {
+__device__ int locate(const MeshDev& m, int owner, Cell<D>& C, bool p0_ok, const double p0[3], const double x[3],
+                      const double disp[3], const double e[3], double w, double cs2, double xi[3], int* nhit,
+                      double* bias) {
   double cur[3] = {x[0], x[1], x[2]};
   double dep[3] = {x[0] + disp[0], x[1] + disp[1], x[2] + disp[2]};
-  int c[3];
-  cell_xyz<D>(m, owner, c);
   int cell = owner;
   double sgn = 1.0;  // current direction = sgn * e
+  double pi[3] = {p0[0], p0[1], p0[2]};
+  bool pi_ok = p0_ok;
   for (int life = 1;; life++) {
     if (life > 50) return -1;
-    double pb[3];
-    const int face = crossed_first<D>(m, c, cur, dep, pb);
-    if (face < 0) break;
+    double pb[3], po[3];
+    const bool po_ok = map_inv<D>(m, C, dep, po);
+    double pc[3] = {po[0], po[1], po[2]};
+    const int face = crossed_first<D>(m, C, cur, dep, pi_ok, pi, po_ok, pc, pb);
+    if (face < 0) {  // dep lies in this cell, po is its inverse image
+      for (int d = 0; d < D; d++) xi[d] = po[d];
+      if (!po_ok) return -3;
+      break;
+    }
     bool wrapped;
     int nc[3];
-    const int nb = neighbor<D>(m, c, face, &wrapped, nc);
+    const int nb = neighbor<D>(m, C.c, face, &wrapped, nc);
     if (nb < 0) {
       sgn = -sgn;
       double vel = 0, dist = 0;
@@ -264,19 +295,18 @@ __device__ int locate(const MeshDev& m, int owner, const double x[3], const doub
       for (int d = 0; d < D; d++) exu += m.wall_u[face][d] * e[d];
       *bias = *bias + 2 * w * 1.0 * exu / cs2;
       (*nhit)++;
-      continue;
+    } else {
+      if (wrapped) {
+        periodic_shift<D>(m, C.c, face, pb);
+        periodic_shift<D>(m, C.c, face, dep);
+      }
+      for (int d = 0; d < 3; d++) cur[d] = pb[d];
+      for (int d = 0; d < 3; d++) C.c[d] = nc[d];
+      C.load(m);
+      cell = nb;
     }
-    if (wrapped) {
-      periodic_shift<D>(m, c, face, pb);
-      periodic_shift<D>(m, c, face, dep);
-    }
-    for (int d = 0; d < 3; d++) cur[d] = pb[d];
-    c[0] = nc[0];
-    c[1] = nc[1];
-    c[2] = nc[2];
-    cell = nb;
+    pi_ok = map_inv<D>(m, C, cur, pi);
   }
-  if (!map_inv<D>(m, c, dep, xi)) return -3;
   for (int d = 0; d < D; d++) {
     clamp01(xi[d]);
     if (xi[d] < 0 || xi[d] > 1) return -3;
@@ -285,27 +315,55 @@ __device__ int locate(const MeshDev& m, int owner, const double x[3], const doub
   return cell;
 }
 
-// One thread per (streamed direction, DoF). dirw holds per streamed direction the
-// scaled velocity (3) and the weight; with walls, flipmask[i] collects bit alpha
-// for a reversed source direction and bit 0 for any hit, bias_out the added value.
+// Streamed directions: displacement -dt c, scaled velocity and weight.
+struct AssembleDirs {
+  double disp[MAXQ - 1][3], dir[MAXQ - 1][3], w[MAXQ - 1];
+};
+
+// Unit coordinates of every DoF in its owner cell, from which the walks of all its directions
+// start (NaN in the first: the inverse map failed).
 template <int D>
-__global__ __launch_bounds__(128) void k_assemble_general(MeshDev m, int64_t n, int Qm1, const double* __restrict__ coords,
-                                   const int* __restrict__ owner, const double* __restrict__ disp /* Qm1 x 3 */,
-                                   const double* __restrict__ dirw /* Qm1 x 4 */, double cs2,
-                                   int* __restrict__ cell_out, double* __restrict__ xi_out,
-                                   unsigned* __restrict__ flipmask, double* __restrict__ bias_out,
-                                   int* __restrict__ status) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * Qm1) return;
-  const int a = (int)(t / n);
-  const int64_t i = t - (int64_t)a * n;
+__global__ __launch_bounds__(128) void k_owner_unit(MeshDev m, int64_t n, const double* __restrict__ coords,
+                                                    const int* __restrict__ owner, double* __restrict__ p0) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
   const double x[3] = {coords[3 * i], coords[3 * i + 1], coords[3 * i + 2]};
-  const double dp[3] = {disp[3 * a], disp[3 * a + 1], disp[3 * a + 2]};
-  const double e[3] = {dirw[4 * a], dirw[4 * a + 1], dirw[4 * a + 2]};
+  Cell<D> C;
+  cell_xyz<D>(m, owner[i], C.c);
+  C.load(m);
+  double p[3];
+  const bool ok = map_inv<D>(m, C, x, p);
+  for (int d = 0; d < D; d++) p0[D * i + d] = ok ? p[d] : __builtin_nan("");
+}
+
+// One thread per (streamed direction, DoF). With walls, flipmask[i] collects bit alpha for a
+// reversed source direction and bit 0 for any hit, bias_out the added value.
+// Bound by the FP64 Newton iterations of the inverse maps (about 6 of some 300 operations each).
+// The walk keeps the departure point's unit coordinates of the cell it ends in and starts from
+// the DoF's own (k_owner_unit, once instead of once per direction): 2.2 maps per record instead of
+// 4.2 at CFL 0.4. 16^3 p=2 D3Q19 perturbed: 284 -> 230 us in all; vertices held in registers over the
+// iterations, or the directions of 64 DoFs by one block, cost more in occupancy than they save.
+template <int D>
+__global__ __launch_bounds__(128) void k_assemble_general(
+    MeshDev m, int64_t n, int Qm1, const double* __restrict__ coords, const int* __restrict__ owner,
+    const double* __restrict__ p0, AssembleDirs dirs, double cs2, int* __restrict__ cell_out,
+    double* __restrict__ xi_out, unsigned* __restrict__ flipmask, double* __restrict__ bias_out,
+    int* __restrict__ status) {
+  const int a = blockIdx.y;
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t t = (int64_t)a * n + i;
+  const double x[3] = {coords[3 * i], coords[3 * i + 1], coords[3 * i + 2]};
+  const double pi[3] = {p0[D * i], p0[D * i + 1], D == 3 ? p0[D * i + D - 1] : 0.0};
+  const int own = owner[i];
+  Cell<D> C;
+  cell_xyz<D>(m, own, C.c);
+  C.load(m);
   double xi[3] = {0, 0, 0};
   int nhit = 0;
   double bias = 0;
-  const int c = locate<D>(m, owner[i], x, dp, e, dirw[4 * a + 3], cs2, xi, &nhit, &bias);
+  const int c =
+      locate<D>(m, own, C, pi[0] == pi[0], pi, x, dirs.disp[a], dirs.dir[a], dirs.w[a], cs2, xi, &nhit, &bias);
   cell_out[t] = c;
   for (int d = 0; d < D; d++) xi_out[t * D + d] = xi[d];
   if (flipmask) {
@@ -467,8 +525,8 @@ int nat_launch_support_points(nat_ctx* ctx) {
   return 0;
 }
 
-int nat_launch_assemble_general(nat_ctx* ctx, const double* d_disp, const double* d_dirw, int* d_cell, double* d_xi,
-                                unsigned* d_flipmask, double* d_bias) {
+int nat_launch_assemble_general(nat_ctx* ctx, double* d_p0, int* d_cell, double* d_xi, unsigned* d_flipmask,
+                                double* d_bias) {
   nat::MeshDev m;
   m.D = ctx->D;
   for (int a = 0; a < 3; a++) {
@@ -479,16 +537,28 @@ int nat_launch_assemble_general(nat_ctx* ctx, const double* d_disp, const double
     for (int d = 0; d < 3; d++) m.wall_u[f][d] = d < ctx->D ? ctx->desc.wall_velocity[f][d] : 0.0;
   m.cartesian = ctx->desc.cartesian;
   m.vert = ctx->d_vert;
-  const int64_t total = ctx->n_dofs * (ctx->Q - 1);
+  nat::AssembleDirs dirs = {};
+  for (int a = 1; a < ctx->Q; a++) {
+    for (int d = 0; d < 3; d++) {
+      dirs.disp[a - 1][d] = ctx->st.dir[a][d] * (-ctx->dt);
+      dirs.dir[a - 1][d] = ctx->st.dir[a][d];
+    }
+    dirs.w[a - 1] = ctx->st.w[a];
+  }
   const int bs = 128;
+  const unsigned nb = (unsigned)((ctx->n_dofs + bs - 1) / bs);
+  const auto launch = [&](auto DD) {
+    constexpr int D = decltype(DD)::value;
+    hipLaunchKernelGGL(nat::k_owner_unit<D>, dim3(nb), dim3(bs), 0, ctx->stream, m, ctx->n_dofs, ctx->d_coords,
+                       ctx->d_owner, d_p0);
+    hipLaunchKernelGGL(nat::k_assemble_general<D>, dim3(nb, ctx->Q - 1), dim3(bs), 0, ctx->stream, m, ctx->n_dofs,
+                       ctx->Q - 1, ctx->d_coords, ctx->d_owner, d_p0, dirs, ctx->st.cs2, d_cell, d_xi, d_flipmask,
+                       d_bias, ctx->d_status);
+  };
   if (ctx->D == 3)
-    hipLaunchKernelGGL(nat::k_assemble_general<3>, dim3((unsigned)((total + bs - 1) / bs)), dim3(bs), 0, ctx->stream,
-                       m, ctx->n_dofs, ctx->Q - 1, ctx->d_coords, ctx->d_owner, d_disp, d_dirw, ctx->st.cs2, d_cell,
-                       d_xi, d_flipmask, d_bias, ctx->d_status);
+    launch(std::integral_constant<int, 3>{});
   else
-    hipLaunchKernelGGL(nat::k_assemble_general<2>, dim3((unsigned)((total + bs - 1) / bs)), dim3(bs), 0, ctx->stream,
-                       m, ctx->n_dofs, ctx->Q - 1, ctx->d_coords, ctx->d_owner, d_disp, d_dirw, ctx->st.cs2, d_cell,
-                       d_xi, d_flipmask, d_bias, ctx->d_status);
+    launch(std::integral_constant<int, 2>{});
   NAT_HIP(hipGetLastError());
   return 0;
 }

@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <new>
 #include <string>
 #include <vector>
@@ -12,8 +13,8 @@
 #include "nat_internal.hpp"
 
 // kernel launchers (k_*.hip)
-int nat_launch_assemble_general(nat_ctx* ctx, const double* d_disp, const double* d_dirw, int* d_cell, double* d_xi,
-                                unsigned* d_flipmask, double* d_bias);
+int nat_launch_assemble_general(nat_ctx* ctx, double* d_p0, int* d_cell, double* d_xi, unsigned* d_flipmask,
+                                double* d_bias);
 int nat_launch_support_points(nat_ctx* ctx);
 int nat_launch_wall_compact(nat_ctx* ctx, const int* d_list, const unsigned* d_flipmask, const double* d_bias);
 int nat_launch_assemble_axis(nat_ctx* ctx, const int* d_N, const double* d_vaxis, int maxc, const double* d_disp,
@@ -172,23 +173,34 @@ void map_cell(const nat_ctx* c, const int cc[3], const double xi[3], bool cartes
 }
 
 double min_vertex_distance(const nat_ctx* c) {
-  double mind = 1e300;
-  const int nv = c->D == 3 ? 8 : 4;
-  const int nz = c->D == 3 ? c->desc.ncells[2] : 1;
+  // every vertex pair of a cell once, by the offset between its two vertices; the square root is
+  // monotone, so one of the smallest square is the smallest distance
+  const int nx = c->desc.ncells[0] + 1, ny = c->desc.ncells[1] + 1, nz = c->D == 3 ? c->desc.ncells[2] + 1 : 1;
+  int off[13][3], no = 0;
+  for (int dz = 0; dz <= (nz > 1 ? 1 : 0); dz++)
+    for (int dy = -1; dy <= 1; dy++)
+      for (int dx = -1; dx <= 1; dx++)
+        if (dz > 0 || dy > 0 || (dy == 0 && dx > 0)) {
+          off[no][0] = dx;
+          off[no][1] = dy;
+          off[no++][2] = dz;
+        }
+  double m2[13];
+  std::fill(m2, m2 + 13, 1e300);
   for (int k = 0; k < nz; k++)
-    for (int j = 0; j < c->desc.ncells[1]; j++)
-      for (int i = 0; i < c->desc.ncells[0]; i++) {
-        int cc[3] = {i, j, k};
-        double V[8][3];
-        for (int v = 0; v < nv; v++) cell_vertex(c, cc, v, V[v]);
-        for (int a = 0; a < nv; a++)
-          for (int b = a + 1; b < nv; b++) {
-            double s = 0;
-            for (int d = 0; d < c->D; d++) s += (V[a][d] - V[b][d]) * (V[a][d] - V[b][d]);
-            mind = std::min(mind, std::sqrt(s));
-          }
+    for (int j = 0; j < ny; j++)
+      for (int i = 0; i < nx; i++) {
+        const double* a = &c->verts[3 * ((size_t)i + (size_t)nx * ((size_t)j + (size_t)ny * k))];
+        for (int o = 0; o < no; o++) {
+          const int i1 = i + off[o][0], j1 = j + off[o][1], k1 = k + off[o][2];
+          if (i1 < 0 || i1 >= nx || j1 < 0 || j1 >= ny || k1 >= nz) continue;
+          const double* b = a + 3 * (off[o][0] + (ptrdiff_t)nx * (off[o][1] + (ptrdiff_t)ny * off[o][2]));
+          double s = 0;
+          for (int d = 0; d < c->D; d++) s += (a[d] - b[d]) * (a[d] - b[d]);
+          if (s < m2[o]) m2[o] = s;
+        }
       }
-  return mind;
+  return std::min(1e300, std::sqrt(*std::min_element(m2, m2 + no)));
 }
 
 // uniform axis-aligned lattice (a prerequisite of the structured backend)
@@ -502,23 +514,12 @@ bool structured_instantiated(int D, int Q, int p) {
   return Q == 9 && pq;
 }
 
-int assemble_general(nat_ctx* ctx) {
+// while_running: host work that may overlap the device's (before the first wait)
+int assemble_general(nat_ctx* ctx, const std::function<void()>& while_running = {}) {
   const int Qm1 = ctx->Q - 1;
-  std::vector<double> disp(3 * Qm1, 0.0), dirw(4 * Qm1, 0.0);
-  for (int a = 1; a < ctx->Q; a++) {
-    for (int d = 0; d < 3; d++) {
-      disp[3 * (a - 1) + d] = ctx->st.dir[a][d] * (-ctx->dt);
-      dirw[4 * (a - 1) + d] = ctx->st.dir[a][d];
-    }
-    dirw[4 * (a - 1) + 3] = ctx->st.w[a];
-  }
   DevScratch tmp;
-  double *ddisp, *ddirw, *dbias = nullptr;
+  double* dbias = nullptr;
   unsigned* dmask = nullptr;
-  TRY(tmp.get(ctx, &ddisp, disp.size()));
-  TRY(tmp.get(ctx, &ddirw, dirw.size()));
-  NAT_HIP(hipMemcpyAsync(ddisp, disp.data(), disp.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-  NAT_HIP(hipMemcpyAsync(ddirw, dirw.data(), dirw.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
   const int64_t nrec = ctx->n_dofs * Qm1;
   if (!ctx->dep_cell) TRY(alloc(ctx, &ctx->dep_cell, nrec));
   if (!ctx->dep_xi64) TRY(alloc(ctx, &ctx->dep_xi64, nrec * ctx->D));
@@ -527,7 +528,9 @@ int assemble_general(nat_ctx* ctx) {
     TRY(tmp.get(ctx, &dbias, nrec));
     NAT_HIP(hipMemsetAsync(dmask, 0, sizeof(unsigned) * ctx->n_dofs, ctx->stream));
   }
-  TRY(nat_launch_assemble_general(ctx, ddisp, ddirw, ctx->dep_cell, ctx->dep_xi64, dmask, dbias));
+  // scratch (D doubles per DoF): the population buffer that the next step writes
+  TRY(nat_launch_assemble_general(ctx, (double*)ctx->f[1 - ctx->cur], ctx->dep_cell, ctx->dep_xi64, dmask, dbias));
+  if (while_running) while_running();
   if (ctx->fp32) {
     if (!ctx->dep_rec32) TRY(alloc(ctx, &ctx->dep_rec32, nrec * (ctx->D + 1)));
     const int64_t nl =
@@ -805,13 +808,16 @@ int nat_set_vertices(nat_ctx* ctx, const double* vertices) {
     return code;
   };
   NAT_HIP(hipMemcpy(ctx->d_vert, ctx->verts.data(), ctx->verts.size() * sizeof(double), hipMemcpyHostToDevice));
-  ctx->h_min = min_vertex_distance(ctx);
-  if (d.scheme != NAT_SL) return 0;  // SEDG evaluates the geometry from the vertices in every stage
+  if (d.scheme != NAT_SL) {  // SEDG evaluates the geometry from the vertices in every stage
+    ctx->h_min = min_vertex_distance(ctx);
+    return 0;
+  }
   {
     const int rc = nat_launch_support_points(ctx);
     if (rc) return restore(rc, ctx->err);
   }
   if (ctx->backend == NAT_BACKEND_STRUCTURED) {
+    ctx->h_min = min_vertex_distance(ctx);
     bool ok = false;
     StructTables t;
     const int rc = build_structured_tables(ctx, t, &ok);
@@ -820,7 +826,7 @@ int nat_set_vertices(nat_ctx* ctx, const double* vertices) {
     commit_structured_tables(ctx, t);
     return 0;
   }
-  const int rc = assemble_general(ctx);
+  const int rc = assemble_general(ctx, [ctx] { ctx->h_min = min_vertex_distance(ctx); });
   if (rc) {
     const std::string msg = ctx->err;
     restore(rc, msg);
