@@ -234,6 +234,21 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t comp_rsrc(const T* p) {
                                            (int)0xffffffffu, 0x00020000);
 }
 
+// Store to p[i] (p uniform), written through to the device (sc1): a wave stores whole lines, and
+// the output leaves the caches while the kernel runs instead of in the write-back at its end
+// (us per step, FP32 and FP64: p=2 128^2 25.9 -> 24.9, 26.2 -> 26.0; 64^2 11.3 -> 11.1,
+// 12.8 -> 11.7; p=3 64^2 18.2 -> 17.8, 22.5 -> 21.2; beyond the Infinity Cache, p=2 256^2,
+// 60.9 -> 60.4, 89 -> 91.5).
+template <typename T>
+__device__ __forceinline__ void comp_store(T* p, int64_t i, T v) {
+  const int off = (int)((unsigned)i * (unsigned)sizeof(T));
+  if constexpr (sizeof(T) == 4)
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), comp_rsrc(p), off, 0, 16);
+  else
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(unsigned __attribute__((ext_vector_type(2))), v),
+                                          comp_rsrc(p), off, 0, 16);
+}
+
 // A row of P + 1 values in the fewest loads of 16, 12, 8 and 4 bytes.
 template <int P, typename T>
 __device__ __forceinline__ void comp_row(__amdgpu_buffer_rsrc_t r, int off, T (&v)[P + 1]) {
@@ -360,8 +375,8 @@ __device__ __forceinline__ void comp_stream_dir(const CompArgs<T>& a, const doub
 // 128^2 p=2 FP32, 9 us at the cache's rate), so the record of the next direction is loaded ahead
 // and the rows come in whole-row loads that no branch splits. Against single loads with the cut
 // terms behind branches and the values kept in LDS, us per step (FP32, FP64; walls in y):
-// p=2 16^2 11.3 -> 9.6, 12.1 -> 9.5; p=2 128^2 29.2 -> 26.0, 33.0 -> 26.6; p=3 64^2 32.2 -> 18.4,
-// 34.9 -> 22.5; p=2 256^2 80.2 -> 61.5, 121 -> 90; Pr 0.71 128^2 40.5 -> 34.2, 44.0 -> 35.7. Also
+// p=2 16^2 11.3 -> 9.6, 12.1 -> 9.3; p=2 128^2 29.2 -> 24.9, 33.0 -> 26.0; p=3 64^2 32.2 -> 17.8,
+// 34.9 -> 21.2; p=2 256^2 80.2 -> 60.4, 121 -> 91.5; Pr 0.71 128^2 40.5 -> 33.1, 44.0 -> 34.3. Also
 // fetching the next direction's rows ahead (156 VGPRs) is faster on 128^2 FP32 without walls
 // (25.1 -> 22.7) and slower elsewhere.
 template <bool PR>
@@ -467,8 +482,8 @@ __global__ __launch_bounds__(CW * 64) void k_sl_comp_wide(CompArgs<T> a, const d
   if (live) nd = comp_node_sums<T>(rho, u0, u1, tf, tg, a);
   if (w == 0 && live && !(nd.rho >= 1e-10)) atomicOr(a.status, 1);
   auto store = [&](int q, double fn, double gn) {
-    a.fout[(int64_t)q * a.stride + i] = (T)(fn - tab[q * CTAB + CT_W] * a.rho0);
-    a.gout[(int64_t)q * a.stride + i] = (T)(gn - tab[q * CTAB + CT_W] * a.gshift);
+    comp_store(a.fout + (int64_t)q * a.stride, i, (T)(fn - tab[q * CTAB + CT_W] * a.rho0));
+    comp_store(a.gout + (int64_t)q * a.stride, i, (T)(gn - tab[q * CTAB + CT_W] * a.gshift));
   };
   CompNeq s;
   if constexpr (PR) {
