@@ -496,17 +496,23 @@ static int launch_push(nat_ctx* ctx, PushArgs<T> a, const CollideArgs<T>& ca, bo
 // Tile of a context: 1 the small one, 2 the large one, 0 where k_sl_struct is faster. While the
 // small tiles leave CUs idle, a step lasts as long as one workgroup does, and less work per
 // workgroup wins; past a few workgroups per CU the share of nodes collided twice (NN over the
-// tile's nodes) and the length of the stored lines decide. Cubic boxes, us per step in k_sl_struct /
-// small / large tile (64 steps, one MI355X):
-//   D3Q27 p=4 FP32   8^3 cells 14.1/ 9.2/11.7   12^3 17.5/13.6/13.3   16^3 21.3/24.9/20.6   32^3 168/203/148
-//             FP64   8^3       16.0/10.3/13.5   12^3 18.8/21.0/18.8   16^3 28.7/40.4/35.6
-//   D3Q19 p=3 FP32   8^3        9.5/ 5.7/ 7.4   16^3 14.4/ 8.8/ 8.8   30^3 65.3/35.9/32.9
-//             FP64   8^3       10.4/ 6.2/ 8.0   16^3 16.1/11.8/13.1   30^3 72.7/52.0/72.0
-//   D3Q27 p=2 FP32   8^3       14.4/ 5.3/11.2   24^3 18.4/12.2/13.3   48^3 73.2/70.8/55.9
-//             FP64   8^3       16.0/ 5.2/11.4   24^3 19.0/13.4/15.7   48^3 121/129/127
-//   D2Q9  p=4 FP32   32^2       5.8/ 4.2/ 4.9   100^2 9.1/ 6.8/ 7.0   256^2 26.1/23.5/19.8
-//             FP64   32^2       6.2/ 4.3/ 5.4   100^2 9.6/ 7.9/ 8.5   128^2 9.5/10.5/10.0
-//   D2Q9  p=2 FP32   64^2       5.7/ 3.3/ 4.0   128^2 5.8/ 4.1/ 4.2   256^2 7.7/ 8.1/ 7.4
+// tile's nodes) and the length of the stored lines decide. k_sl_struct pays whole rounds of 256
+// tiles of 1024 nodes, so it is at its best where a mesh fills one (p=4 16^3, p=2 32^3 cells).
+// Cubic boxes, us per step in k_sl_struct / small / large tile (runs of 32 to 100 steps on a warm
+// card, one MI355X; -: no such tile):
+//   D3Q27 p=4 FP32   8^3 cells 14.1/ 9.2/11.8   12^3 17.4/14.3/13.8   16^3 20.8/25.0/20.3   30^3 221/171/139
+//             FP64   8^3       16.0/10.3/ -     11^3 21.3/20.0/ -     12^3 18.8/21.3/ -     16^3 28.4/40.7/ -
+//   D3Q19 p=4 FP32   8^3        9.4/ 7.0/ 8.4   12^3 11.0/10.0/ 9.1   16^3 13.4/18.5/14.0   24^3 47.8/56.2/42.2
+//             FP64   8^3       10.1/ 7.7/ -     11^3 14.3/11.8/ -     12^3 12.5/12.8/ -     16^3 18.5/24.3/ -
+//   D3Q19 p=3 FP32  16^3       13.9/ 8.7/ 8.7   21^3 32.5/16.7/14.8   32^3 66.5/41.1/37.9
+//             FP64  24^3       35.1/30.1/ -     28^3 57.5/39.9/ -     32^3 83.9/78.0/ -
+//   D3Q27 p=2 FP32  16^3       15.1/ 6.2/11.7   30^3 22.4/18.1/20.0   32^3 20.3/23.1/19.5   48^3 75.8/78.3/64.6
+//             FP64  16^3       16.3/ 6.6/ -     30^3 26.6/23.2/ -     32^3 26.6/29.1/ -     40^3 60.0/48.0/ -
+//   D3Q19 p=2 FP32  24^3       12.4/ 8.6/ 9.6   30^3 15.6/13.3/14.6   32^3 14.1/16.1/14.1   48^3 50.8/49.2/44.4
+//             FP64  30^3       17.9/16.2/ -     32^3 17.7/18.7/ -     40^3 39.0/32.6/ -     48^3 65.5/73.9/ -
+//   D2Q9  p=4 FP32   32^2       5.8/ 4.2/ 4.9   100^2 8.9/ 6.5/ 6.9   128^2 7.5/ 8.3/ 7.3   256^2 26.1/23.5/19.8
+//             FP64   32^2       6.2/ 4.3/ -     100^2 9.6/ 7.7/ -     128^2 9.5/10.5/ -
+//   D2Q9  p=2 FP32   64^2       5.7/ 3.3/ 4.0   128^2 5.6/ 4.0/ 4.1   256^2 7.6/ 7.7/ 7.0
 static int push_tile(const nat_ctx* ctx) {
   const int64_t cells = (int64_t)ctx->desc.ncells[0] * ctx->desc.ncells[1] * (ctx->D == 3 ? ctx->desc.ncells[2] : 1);
   if (ctx->D == 2) {
@@ -514,9 +520,14 @@ static int push_tile(const nat_ctx* ctx) {
     if (ctx->p == 3) return 1;
     return cells <= 10240 ? 1 : (ctx->fp32 ? 2 : 0);
   }
-  if (ctx->p == 2) return cells <= 16384 ? 1 : (ctx->fp32 ? 2 : (ctx->Q == 27 && cells > 65536 ? 0 : 1));
+  if (ctx->p == 2) {
+    if (ctx->fp32) return cells <= 28672 ? 1 : 2;
+    return cells <= 28672 || (cells > 32768 && cells < 65536) ? 1 : 0;
+  }
   if (ctx->p == 3) return ctx->fp32 && cells > 8192 ? 2 : 1;
-  return cells <= 1024 ? 1 : (ctx->fp32 ? 2 : 0);
+  if (!ctx->fp32) return cells <= 1400 ? 1 : 0;
+  if (cells <= 1024) return 1;
+  return ctx->Q == 19 && cells > 3375 && cells <= 4096 ? 0 : 2;
 }
 
 template <typename T>

@@ -309,12 +309,14 @@ void dg_points(const nat_ctx* c, std::vector<double>& xyz) {
       }
 }
 
-// Elements between the arrays of two directions: whole 512-byte lines, and not a multiple of 1 MiB,
-// which puts the same node of all directions on one memory channel (2,097,152 nodes in FP32,
-// D3Q27 p = 4: 180 us per step at 8 MiB, 147 with 16,640 bytes more).
-int64_t pop_stride(int64_t n, int64_t es) {
+// Elements between the arrays of two directions: whole 512-byte lines, and in FP32 or 2D not a
+// multiple of 1 MiB, which puts the same node of all directions on one memory channel (2,097,152
+// nodes in FP32, D3Q27 p = 4: 180 us per step at 8 MiB, 147 with 16,640 bytes more; 512^2 nodes in
+// FP64, D2Q9 p = 2: 9.5 -> 8.9). FP64 in 3D gains nothing (D3Q27 p = 4, 64^3 nodes: 26.95 -> 27.15,
+// 128^3: 268 -> 270).
+int64_t pop_stride(int64_t n, int64_t es, int D) {
   const int64_t s = (n + 127) / 128 * 128;
-  return s * es % (1 << 20) == 0 ? s + 16640 / es : s;
+  return (es == 4 || D == 2) && s * es % (1 << 20) == 0 ? s + 16640 / es : s;
 }
 
 // device storage index of FE_Q DoF (i,j,k)
@@ -731,7 +733,7 @@ int nat_create(const nat_desc* desc, nat_ctx** out) {
     ctx->backend = NAT_BACKEND_GENERAL;
   }
   const size_t es = ctx->fp32 ? sizeof(float) : sizeof(double);
-  ctx->stride = pop_stride(ctx->n_store, es);
+  ctx->stride = pop_stride(ctx->n_store, es, ctx->D);
   for (int b = 0; b < 2; b++) {
     hipError_t e = hipMalloc(&ctx->f[b], es * ctx->stride * ctx->Q);
     if (e != hipSuccess) return fail(ctx, NAT_ERR_NOMEM, "device allocation of populations failed");
@@ -1395,7 +1397,7 @@ int64_t nat_internal_footprint(const nat_desc* d) {
   int64_t n_store, recs = 0;
   if (d->scheme != NAT_SL) {
     n_store = ncell * (D == 3 ? np * np * np : np * np);
-    recs = Q * pop_stride(n_store, es) * es;  // RK5 df
+    recs = Q * pop_stride(n_store, es, D) * es;  // RK5 df
   } else {
     bool walls = false;
     for (int a = 0; a < D; a++) walls = walls || !d->periodic[a];
@@ -1410,7 +1412,7 @@ int64_t nat_internal_footprint(const nat_desc* d) {
       if (walls) recs += 4 * nfe + nfe * (4 + 8 * Q) + 4 * nfe + (int64_t)(Q - 1) * nfe * 8;
     }
   }
-  const int64_t stride = pop_stride(n_store, es);
+  const int64_t stride = pop_stride(n_store, es, D);
   int64_t bytes = 2 * Q * stride * es * (d->compressible ? 2 : 1);
   bytes += (1 + D) * n_store * es + (d->compressible ? 2 * 8 * n_store : 0);
   bytes += recs;
