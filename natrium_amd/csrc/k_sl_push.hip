@@ -575,13 +575,21 @@ static int push_typed(nat_ctx* ctx, bool col) {
 
 }  // namespace nat
 
-// Whether runs of several steps of this context take the collide-then-stream form: symmetric
+// Whether a run of nsteps steps of this context takes the collide-then-stream form: symmetric
 // one-dimensional tables at p = 2-4, populations within 32-bit buffer offsets, and a tile that is
-// faster than k_sl_struct's.
-bool nat_push_eligible(const nat_ctx* ctx) {
-  return ctx->desc.scheme == NAT_SL && !ctx->desc.compressible && ctx->backend == NAT_BACKEND_STRUCTURED &&
-         ctx->ax_sym && ctx->ax_w && ctx->p >= 2 && ctx->p <= 4 &&
-         ctx->stride * (ctx->fp32 ? 4 : 8) * ctx->Q < (int64_t)0xffffffffu && nat::push_tile(ctx) > 0;
+// faster than k_sl_struct's. On a mesh that fills one or two rounds of k_sl_struct's tiles exactly
+// (p=4 16^3, p=2 32^3) the two are close, and the run must be long: from an idle card the first
+// hundred launches are slower here (D3Q27 p=4 16^3 FP32, k_sl_struct / k_sl_push in us per step:
+// 16 steps 21.8/23.3, 64 20.5/20.8, 128 20.6/20.0, 1000 20.9/19.9).
+bool nat_push_eligible(const nat_ctx* ctx, int nsteps) {
+  if (nsteps < 2 || ctx->desc.scheme != NAT_SL || ctx->desc.compressible || ctx->backend != NAT_BACKEND_STRUCTURED ||
+      !ctx->ax_sym || !ctx->ax_w || ctx->p < 2 || ctx->p > 4 ||
+      ctx->stride * (ctx->fp32 ? 4 : 8) * ctx->Q >= (int64_t)0xffffffffu)
+    return false;
+  const int tile = nat::push_tile(ctx);
+  const int64_t round = 256 * 1024;
+  const bool close = ctx->D == 3 && tile == 2 && ctx->n_store % round == 0 && ctx->n_store <= 2 * round;
+  return tile > 0 && (!close || nsteps >= 96);
 }
 
 // One launch from f[cur] into f[1 - cur]: collide (when col) and stream.

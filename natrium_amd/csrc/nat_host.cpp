@@ -27,7 +27,7 @@ int nat_internal_pack_step(nat_ctx* const* ctxs, int n, int nsteps, hipStream_t 
 int nat_internal_autotune(nat_ctx* ctx, int nsteps, int* tile, double* best_us);
 int nat_internal_autotune_general(nat_ctx* ctx, int nsteps, int* tile, double* best_us);
 int nat_launch_sl_general(nat_ctx* ctx, int write_macro);
-bool nat_push_eligible(const nat_ctx* ctx);
+bool nat_push_eligible(const nat_ctx* ctx, int nsteps);
 int nat_launch_sl_push(nat_ctx* ctx, bool col);
 int nat_launch_collide(nat_ctx* ctx, int init);
 int nat_launch_collide_step(nat_ctx* ctx, bool macro);
@@ -574,7 +574,7 @@ int assemble_general(nat_ctx* ctx, const std::function<void()>& while_running = 
 }
 
 void nat_drop_graphs(nat_ctx* ctx) {
-  for (int b = 0; b < 2; b++) {
+  for (int b = 0; b < 4; b++) {
     if (ctx->gexec[b]) hipGraphExecDestroy(ctx->gexec[b]);
     if (ctx->graph[b]) hipGraphDestroy(ctx->graph[b]);
     ctx->gexec[b] = nullptr;
@@ -1068,12 +1068,10 @@ int nat_stabilize(nat_ctx* ctx) {
   return check_status(ctx);
 }
 
-// Runs of at least this many steps of a structured context take the collide-then-stream form
-// (k_sl_push.hip): n steps are one streaming launch, n - 1 launches that collide and stream, and
-// one collision, n + 1 in all. A single step would be two launches, and is one of the fused
+// Runs of two steps or more of a structured context take the collide-then-stream form where it is
+// the faster (nat_push_eligible, k_sl_push.hip): n steps are one streaming launch, n - 1 launches
+// that collide and stream, and one collision, n + 1 in all. A single step would be two launches, and is one of the fused
 // stream-then-collide kernel instead.
-static constexpr int kPushSteps = 2;
-
 static int push_launch(nat_ctx* ctx, int n, bool col) {
   for (int s = 0; s < n; s++) {
     TRY(nat_launch_sl_push(ctx, col));
@@ -1084,7 +1082,7 @@ static int push_launch(nat_ctx* ctx, int n, bool col) {
 
 static int step_launch(nat_ctx* ctx, int nsteps, bool macro_last = true) {
   if (!ctx->assembled) return fail(ctx, NAT_ERR_STATE, "operator not assembled");
-  if (nsteps >= kPushSteps && nat_push_eligible(ctx)) {
+  if (nat_push_eligible(ctx, nsteps)) {
     TRY(push_launch(ctx, 1, false));
     TRY(push_launch(ctx, nsteps - 1, true));
     return nat_launch_collide_step(ctx, macro_last);
@@ -1152,12 +1150,12 @@ extern "C++" int nat_internal_capture(nat_ctx* ctx, int nsteps, bool macro_last,
 
 static int step_enqueue(nat_ctx* ctx, int nsteps) {
   int left = nsteps;
-  const bool push = ctx->assembled && nsteps >= kPushSteps && nat_push_eligible(ctx);
+  const bool push = ctx->assembled && nat_push_eligible(ctx, nsteps);
   // collide-then-stream: the streaming of the first step, then graphs of (collide; stream)
   if (push) TRY(push_launch(ctx, 1, false));
   // the last step writes the macroscopic fields and always runs as a plain launch
   while (ctx->use_graphs && left - 1 >= kGraphSteps) {
-    const int par = ctx->cur;
+    const int par = ctx->cur + (push ? 2 : 0);
     if (!ctx->gexec[par]) {
       hipGraph_t g = nullptr;
       TRY(capture(ctx, &g, [&] {

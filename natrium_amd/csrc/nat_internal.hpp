@@ -176,9 +176,9 @@ struct nat_ctx {
   int64_t n_wall = 0;
   bool has_walls = false;
 
-  // captured step chunks, one per starting ping-pong buffer
-  hipGraph_t graph[2] = {nullptr, nullptr};
-  hipGraphExec_t gexec[2] = {nullptr, nullptr};
+  // captured step chunks, one per starting ping-pong buffer; the last two: of collide-then-stream launches
+  hipGraph_t graph[4] = {};
+  hipGraphExec_t gexec[4] = {};
   bool use_graphs = true;
 
   // residuals of the results table: fields of the previous 100th-iteration call

@@ -49,6 +49,7 @@ def _solver(stencil, N, p, precision, stabilizer=False):
     ("D3Q27", [27, 25, 26], 2, 2, False),
     ("D3Q27", [31, 31, 30], 2, 2, False),  # large tile (FP32)
     ("D3Q19", [34, 33, 31], 2, 2, True),   # small tile past one round (FP64)
+    ("D3Q27", [16, 16, 16], 4, 96, False),  # exactly one round of the fused kernel: long runs only (FP32)
     ("D3Q19", [11, 11, 11], 4, 2, False),  # small tile (FP64), large (FP32)
     ("D3Q19", [4, 2, 2], 3, 3, False),
     ("D3Q27", [5, 3, 2], 3, 3, False),
