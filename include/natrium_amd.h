@@ -245,6 +245,15 @@ int nat_autotune(nat_ctx* ctx, int nsteps, int* tile /* 3, may be NULL */);
  * NAT_ERR_ARG for another value or backend. */
 int nat_set_general_form(nat_ctx* ctx, int form);
 
+/* Form of the step kernel where a context has several, no counterpart in the reference: all forms
+ * give bit-identical populations and fields and differ in the sizes they serve and in time.
+ *   compressible: 1 reads a direction and its opposite at 32-bit offsets, 0 at 64-bit addresses
+ *     (always available; the rule takes it for arrays of more than 4/3 GiB).
+ * nat_set_step_form pins one (-1: the rule); NAT_ERR_ARG for a form this context does not have.
+ * nat_step_form returns the form a run of nsteps >= 1 steps takes. */
+int nat_set_step_form(nat_ctx* ctx, int form);
+int nat_step_form(nat_ctx* ctx, int nsteps, int* form);
+
 /* ---- Output and restart (host side, from fields downloaded through this API) ---- */
 
 /* One row of the reference's results table: SolverStats::update/printNewLine

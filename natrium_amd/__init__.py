@@ -59,6 +59,7 @@ EXPORTS = [
     "nat_step_timed", "nat_get_macro", "nat_get_knudsen", "nat_sums", "nat_sums_noalloc", "nat_sync",
     "nat_stats", "nat_write_stats", "nat_write_vtu", "nat_checkpoint_write", "nat_checkpoint_read",
     "nat_struct_tile", "nat_pack_key", "nat_step_packed", "nat_autotune", "nat_set_general_form",
+    "nat_set_step_form", "nat_step_form",
 ]
 
 _lib = None
@@ -140,6 +141,10 @@ def lib():
     L.nat_autotune.argtypes = [vp, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
     L.nat_set_general_form.restype = ctypes.c_int
     L.nat_set_general_form.argtypes = [vp, ctypes.c_int]
+    L.nat_set_step_form.restype = ctypes.c_int
+    L.nat_set_step_form.argtypes = [vp, ctypes.c_int]
+    L.nat_step_form.restype = ctypes.c_int
+    L.nat_step_form.argtypes = [vp, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
     _lib = L
     return L
 
@@ -396,6 +401,16 @@ class Solver:
         """Pin the general backend's kernel form (nat_set_general_form): -1 default rule,
         0 eight waves per block, 1 sixteen waves per block (FP32 storage, 3D)."""
         self._check(lib().nat_set_general_form(self._h, int(form)))
+
+    def set_step_form(self, form):
+        """Pin the step kernel's form (nat_set_step_form), -1: the rule."""
+        self._check(lib().nat_set_step_form(self._h, int(form)))
+
+    def step_form(self, nsteps=1):
+        """The kernel form that a run of nsteps steps takes (nat_step_form)."""
+        f = ctypes.c_int(0)
+        self._check(lib().nat_step_form(self._h, int(nsteps), ctypes.byref(f)))
+        return f.value
 
 
 def step_packed(solvers, nsteps):

@@ -19,6 +19,9 @@
 // equilibria at rest with T = 1; the collision un-shifts in FP64.
 #include "nat_collide.hpp"
 #include "nat_fastdiv.hpp"
+#include "nat_offsets.hpp"
+
+int nat_comp_form(const nat_ctx* ctx, int form = -1);
 
 namespace nat {
 
@@ -222,9 +225,11 @@ __device__ __forceinline__ CompRec comp_record(const CompArgs<T>& a, int al, int
   return {a.cell[r], x.x, x.y};
 }
 
-// Buffer resource from a direction's array on, for 32-bit byte offsets (uniform base). Opposite
-// directions are two arrays apart and an array is below 2 GiB (the records of a larger mesh do
-// not fit the device), so offsets into either stay below 2^32.
+// Buffer resource from a direction's array on, for 32-bit byte offsets (uniform base). The rows of
+// a direction and of its opposite are read from the lower one's array on, which takes arrays of at
+// most 4/3 GiB (pair_offsets_fit, opposite directions are two arrays apart; in FP64 178,956,970
+// DoFs, 241 GB of context). The stores stay within one array, below 2 GiB on any mesh whose
+// populations and records fit the device.
 template <typename T>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t comp_rsrc(const T* p) {
   const uint64_t pb = (uint64_t)p;
@@ -289,7 +294,8 @@ __device__ __forceinline__ double comp_min_abs(double a, double b) {
 // whole; where a product weight is under the cut-off (on the Cartesian meshes every lane of the
 // directions along an axis) the terms are dropped by selects, not by branches around their loads.
 // Lanes whose path was reflected at a wall read the opposite direction's array.
-template <int Q, int P, typename T>
+// FAR: arrays beyond the 32-bit offsets, read through 64-bit addresses instead.
+template <int Q, int P, typename T, bool FAR>
 __device__ __forceinline__ void comp_stream_dir(const CompArgs<T>& a, const double* __restrict__ tab, int64_t i,
                                                 int al, int widx, unsigned wmask, const CompRec& rec, double& fo,
                                                 double& go) {
@@ -310,10 +316,10 @@ __device__ __forceinline__ void comp_stream_dir(const CompArgs<T>& a, const doub
     af = 0;
     ag = 0;
     // one resource over the direction and its opposite: a reflected lane adds their distance
-    const int lo = al < a.opp[al] ? al : a.opp[al];
+    const int sd = flip ? a.opp[al] : al, lo = al < a.opp[al] ? al : a.opp[al];
     const __amdgpu_buffer_rsrc_t rf = comp_rsrc(a.fin + (int64_t)lo * a.stride),
                                  rg = comp_rsrc(a.gin + (int64_t)lo * a.stride);
-    const unsigned src = (unsigned)((flip ? a.opp[al] : al) - lo) * (unsigned)(a.stride * (int64_t)sizeof(T));
+    const unsigned src = (unsigned)(sd - lo) * (unsigned)(a.stride * (int64_t)sizeof(T));
     double mnx = comp_min_abs(lx[0], lx[1]), mny = comp_min_abs(ly[0], ly[1]);
 #pragma unroll
     for (int m = 2; m <= P; m++) {
@@ -327,9 +333,18 @@ __device__ __forceinline__ void comp_stream_dir(const CompArgs<T>& a, const doub
       T vf[ny][P + 1], vg[ny][P + 1];
 #pragma unroll
       for (int y = 0; y < ny; y++) {
-        const int off = (int)(src + (unsigned)(base + n0 * (y0 + y)) * (unsigned)sizeof(T));
-        comp_row<P, T>(rf, off, vf[y]);
-        comp_row<P, T>(rg, off, vg[y]);
+        if constexpr (FAR) {
+          const int64_t k = (int64_t)sd * a.stride + base + n0 * (y0 + y);
+#pragma unroll
+          for (int m = 0; m <= P; m++) {
+            vf[y][m] = a.fin[k + m];
+            vg[y][m] = a.gin[k + m];
+          }
+        } else {
+          const int off = (int)(src + (unsigned)(base + n0 * (y0 + y)) * (unsigned)sizeof(T));
+          comp_row<P, T>(rf, off, vf[y]);
+          comp_row<P, T>(rg, off, vg[y]);
+        }
       }
       if (!cut) {
         // no product weight reaches the cut-off: every term is taken
@@ -386,7 +401,7 @@ constexpr int comp_classes() {
 // ST = false: no streaming, each DoF's own populations are collided in place (the
 // initial collision of CFDSolver::run; fin and fout may be the same arrays, since every
 // value is read before it is written and only this block touches its 64 DoFs).
-template <int Q, int P, typename T, bool PR, bool ST = true, int CW = comp_classes<PR>()>
+template <int Q, int P, typename T, bool PR, bool ST = true, int CW = comp_classes<PR>(), bool FAR = false>
 __global__ __launch_bounds__(CW * 64) void k_sl_comp_wide(CompArgs<T> a, const double* __restrict__ tab,
                                                           int write_macro) {
   constexpr int CL = comp_classes<PR>(), NC = CL / CW;  // a wave holds NC classes
@@ -422,7 +437,7 @@ __global__ __launch_bounds__(CW * 64) void k_sl_comp_wide(CompArgs<T> a, const d
       if (ST && q > 0) {
         const CompRec rec = next;  // the next direction's record is loaded ahead of this one's stencil
         if (q + CW < Q) next = comp_record<T>(a, q + CW, i);
-        comp_stream_dir<Q, P, T>(a, tab, i, q, widx, wmask, rec, fv[k], gv[k]);
+        comp_stream_dir<Q, P, T, FAR>(a, tab, i, q, widx, wmask, rec, fv[k], gv[k]);
         if (so) {
           a.fout[(int64_t)q * a.stride + i] = (T)(fv[k] - tab[q * CTAB + CT_W] * a.rho0);
           a.gout[(int64_t)q * a.stride + i] = (T)(gv[k] - tab[q * CTAB + CT_W] * a.gshift);
@@ -542,6 +557,14 @@ __global__ __launch_bounds__(CW * 64) void k_sl_comp_wide(CompArgs<T> a, const d
   if (write_macro && w == 0 && live) comp_write_macro<T>(a, nd, s.kn, Q, i);
 }
 
+static int opposite_of(const nat_ctx* ctx, int q) {
+  for (int r = 0; r < ctx->Q; r++)
+    if (ctx->st.dir[r][0] == -ctx->st.dir[q][0] && ctx->st.dir[r][1] == -ctx->st.dir[q][1] &&
+        ctx->st.dir[r][2] == -ctx->st.dir[q][2])
+      return r;
+  return q;
+}
+
 template <typename T>
 static void fill_comp(nat_ctx* ctx, CompArgs<T>& a, int src, int dst) {
   a.fin = (const T*)ctx->f[src];
@@ -560,12 +583,7 @@ static void fill_comp(nat_ctx* ctx, CompArgs<T>& a, int src, int dst) {
   a.wall_idx = ctx->has_walls ? ctx->wall_idx : nullptr;
   a.wall_flip = ctx->wall_flip;
   a.wall_bias = ctx->wall_bias;
-  for (int q = 0; q < MAXQ; q++) a.opp[q] = q;
-  for (int q = 0; q < ctx->Q; q++)
-    for (int r = 0; r < ctx->Q; r++)
-      if (ctx->st.dir[r][0] == -ctx->st.dir[q][0] && ctx->st.dir[r][1] == -ctx->st.dir[q][1] &&
-          ctx->st.dir[r][2] == -ctx->st.dir[q][2])
-        a.opp[q] = r;
+  for (int q = 0; q < MAXQ; q++) a.opp[q] = q < ctx->Q ? opposite_of(ctx, q) : q;
   double x[MAXP + 1], w[MAXP + 1];
   gll_points(ctx->p, x, w);
   for (int j = 0; j <= MAXP; j++) {
@@ -622,18 +640,24 @@ static int step_comp(nat_ctx* ctx, int mode) {
   const int write_macro = (mode & STEP_MACRO) ? 1 : 0;
   const unsigned grid = (unsigned)((a.n + 63) / 64);
   const double* tab = ctx->comp_tab;
-  const auto launch = [&](auto PP, auto PR, auto CW) {
-    hipLaunchKernelGGL((k_sl_comp_wide<25, decltype(PP)::value, T, decltype(PR)::value, true, decltype(CW)::value>),
+  const bool far = nat_comp_form(ctx) == 0;
+  const auto launch = [&](auto PP, auto PR, auto CW, auto FAR) {
+    hipLaunchKernelGGL((k_sl_comp_wide<25, decltype(PP)::value, T, decltype(PR)::value, true, decltype(CW)::value,
+                                       decltype(FAR)::value>),
                        dim3(grid), dim3(decltype(CW)::value * 64), 0, ctx->stream, a, tab, write_macro);
   };
   const auto pick = [&](auto PP) {
     using std::integral_constant;
-    if (a.prandtl_set)
-      launch(PP, std::true_type{}, integral_constant<int, 4>{});
+    using four = integral_constant<int, 4>;
+    if (far)  // a mesh of millions of blocks (or the caller's choice)
+      a.prandtl_set ? launch(PP, std::true_type{}, four{}, std::true_type{})
+                    : launch(PP, std::false_type{}, four{}, std::true_type{});
+    else if (a.prandtl_set)
+      launch(PP, std::true_type{}, four{}, std::false_type{});
     else if (grid <= comp_blocks8<T>(decltype(PP)::value))
-      launch(PP, std::false_type{}, integral_constant<int, 8>{});
+      launch(PP, std::false_type{}, integral_constant<int, 8>{}, std::false_type{});
     else
-      launch(PP, std::false_type{}, integral_constant<int, 4>{});
+      launch(PP, std::false_type{}, four{}, std::false_type{});
   };
   switch (ctx->p) {
     case 1:
@@ -718,6 +742,16 @@ int nat_comp_setup(nat_ctx* ctx) {
   if (!ctx->comp_tab) NAT_HIP(hipMalloc(&ctx->comp_tab, t.size() * sizeof(double)));
   NAT_HIP(hipMemcpy(ctx->comp_tab, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
   return 0;
+}
+
+// Form of the compressible step: 1 with 32-bit offsets into a pair of opposite directions, 0 with
+// 64-bit addresses, for arrays beyond them. form: -1 the context's choice, else whether it exists.
+int nat_comp_form(const nat_ctx* ctx, int form) {
+  int apart = 0;
+  for (int q = 0; q < ctx->Q; q++) apart = std::max(apart, std::abs(nat::opposite_of(ctx, q) - q));
+  const bool fit = nat::pair_offsets_fit(apart, ctx->stride, ctx->fp32 ? 4 : 8);
+  if (form >= 0) return form == 0 || (form == 1 && fit);
+  return fit && ctx->form_pref != 0 ? 1 : 0;
 }
 
 int nat_launch_sl_comp(nat_ctx* ctx, int write_macro) {

@@ -24,6 +24,7 @@
 // At 24^3 FP32 the 1.7 GB of a step take 250-340 us between the cache's rate (6.7 TB/s) and
 // memory's (5.0); the small meshes are 5 launches of a serial chain each (vertices, inverse
 // Jacobian, 4 or 9 pairs).
+#include "nat_offsets.hpp"
 #include "nat_sedg.hpp"
 namespace nat {
 
@@ -296,7 +297,7 @@ static void launch_pair(nat_ctx* ctx, const SedgArgs<T>& s, const CollideArgs<T>
 template <typename T>
 bool nat_sedg_pair_stage(nat_ctx* ctx, const SedgArgs<T>& s, const CollideArgs<T>& ca, int collide, int wm) {
   // opposite directions are at most two arrays apart
-  if (3 * s.stride * (int64_t)sizeof(T) > 0xfffffff0ll) return false;
+  if (!pair_offsets_fit(2, s.stride, sizeof(T))) return false;
   const int Q = ctx->Q, P = ctx->p;
 #define NAT_SP(DD, QQ, PP)                              \
   if (Q == QQ && P == PP) {                             \

@@ -40,6 +40,7 @@ int nat_sedg_step(nat_ctx* ctx, int collide_after, int write_macro);
 int nat_comp_setup(nat_ctx* ctx);
 int nat_launch_sl_comp(nat_ctx* ctx, int write_macro);
 int nat_launch_collide_comp(nat_ctx* ctx);
+int nat_comp_form(const nat_ctx* ctx, int form);
 
 namespace nat {
 
@@ -1346,6 +1347,25 @@ int nat_set_general_form(nat_ctx* ctx, int form) {
   if (form < -1 || form > (two ? 1 : 0)) return fail(ctx, NAT_ERR_ARG, "nat_set_general_form: form out of range");
   if (form != ctx->gen_pref) nat_drop_graphs(ctx);  // captured steps hold the other form's launches
   ctx->gen_pref = form;
+  return 0;
+}
+
+int nat_set_step_form(nat_ctx* ctx, int form) {
+  bool ok = form == -1;
+  if (ctx->desc.compressible)
+    ok = ok || nat_comp_form(ctx, form);
+  else
+    return fail(ctx, NAT_ERR_ARG, "nat_set_step_form: the step of this context has no forms");
+  if (form < -1 || !ok) return fail(ctx, NAT_ERR_ARG, "nat_set_step_form: no such form on this mesh");
+  if (form != ctx->form_pref) nat_drop_graphs(ctx);  // captured steps hold the other form's launches
+  ctx->form_pref = form;
+  return 0;
+}
+
+int nat_step_form(nat_ctx* ctx, int nsteps, int* form) {
+  if (!form || nsteps < 1) return fail(ctx, NAT_ERR_ARG, "nat_step_form: a run of steps and a result are needed");
+  if (!ctx->desc.compressible) return fail(ctx, NAT_ERR_ARG, "nat_step_form: the step of this context has no forms");
+  *form = nat_comp_form(ctx, -1);
   return 0;
 }
 
