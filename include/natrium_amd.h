@@ -248,7 +248,9 @@ int nat_set_general_form(nat_ctx* ctx, int form);
 /* Form of the step kernel where a context has several, no counterpart in the reference: all forms
  * give bit-identical populations and fields and differ in the sizes they serve and in time.
  *   compressible: 1 reads a direction and its opposite at 32-bit offsets, 0 at 64-bit addresses
- *     (always available; the rule takes it for arrays of more than 4/3 GiB).
+ *     (always available; the rule takes it for arrays of more than 4/3 GiB);
+ *   SEDG: 1 works on opposite directions in pairs (upwind flux, arrays up to 4/3 GiB; the rule),
+ *     0 on one direction at a time.
  * nat_set_step_form pins one (-1: the rule); NAT_ERR_ARG for a form this context does not have.
  * nat_step_form returns the form a run of nsteps >= 1 steps takes. */
 int nat_set_step_form(nat_ctx* ctx, int form);

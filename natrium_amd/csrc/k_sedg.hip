@@ -36,6 +36,7 @@
 // FP32 storage keeps f~ = f - w rho0 in FP32. L annihilates constants for the
 // upwind flux; for the central flux L(w rho0) = w rho0 sum_a s_a G_a / w_a(i) is
 // added back explicitly. All arithmetic is FP64.
+#include "nat_offsets.hpp"
 #include "nat_sedg.hpp"
 
 namespace nat {
@@ -239,7 +240,7 @@ static int launch_stage(nat_ctx* ctx, const SedgArgs<T>& s, const CollideArgs<T>
 template <typename T>
 static int dispatch_stage(nat_ctx* ctx, const SedgArgs<T>& s, const CollideArgs<T>& ca, int collide, int wm) {
   const int Q = ctx->Q, P = ctx->p;
-  if (!s.central && nat_sedg_pair_stage<T>(ctx, s, ca, collide, wm)) {
+  if (nat_sedg_pair_stage<T>(ctx, s, ca, collide, wm)) {
     NAT_HIP(hipGetLastError());
     return 0;
   }
@@ -354,6 +355,15 @@ int nat_sedg_setup(nat_ctx* ctx) {
     NAT_HIP(hipMemset(ctx->sedg_df, 0, es * ctx->stride * ctx->Q));
   }
   return 0;
+}
+
+// Form of the stage: 1 in opposite pairs (upwind flux; opposite directions are at most two arrays
+// apart), 0 one direction at a time. form: -1 the context's choice, else whether it exists.
+int nat_sedg_form(const nat_ctx* ctx, int form) {
+  const bool pairs =
+      ctx->desc.scheme == NAT_SEDG && nat::pair_offsets_fit(2, ctx->stride, ctx->fp32 ? 4 : 8);
+  if (form >= 0) return form == 0 || (form == 1 && pairs);
+  return pairs && ctx->form_pref != 0 ? 1 : 0;
 }
 
 int nat_sedg_step(nat_ctx* ctx, int collide_after, int write_macro) {

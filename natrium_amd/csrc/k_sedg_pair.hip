@@ -210,7 +210,7 @@ __global__ __launch_bounds__((SedgShape<D, P>::NT)) void k_sedg_pair(SedgArgs<T>
     __builtin_amdgcn_sched_barrier(0);
     const double va = (double)rown[r].va, vo = (double)rown[r].vo;
     buf[k & 1][tid] = make_double2(va, vo);
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    sedg_barrier();
     double la = 0, lo = 0;
 #pragma unroll
     for (int d = 0; d < D; d++) {
@@ -229,7 +229,6 @@ __global__ __launch_bounds__((SedgShape<D, P>::NT)) void k_sedg_pair(SedgArgs<T>
 #pragma unroll
     for (int a = 0; a < D; a++) {
       const double c = fac[a] * rG[r][a];
-      const double ca_ = fmin(c, 0.0), co = fmin(-c, 0.0);  // the upwind one's flux, 0 for the other
       double na = (double)rnb[r][a], no = na, cwu = 0.0;
       if (WALLS && wallf[a] >= 0) {
         na = vo;
@@ -243,8 +242,10 @@ __global__ __launch_bounds__((SedgShape<D, P>::NT)) void k_sedg_pair(SedgArgs<T>
         if (e2 != 0) eu += e2 * uw[2];
         cwu = c * L::w[al] * (3.0 * eu / sc);
       }
-      la = fma(ca_, va - na, la);
-      lo = fma(co, vo - no, lo);
+      // the face belongs to the one of the two for which it is upwind: for the other na or no is its
+      // partner's value, and a flux of zero times it would hand on infinities
+      la = c < 0.0 ? fma(c, va - na, la) : la;
+      lo = c > 0.0 ? fma(-c, vo - no, lo) : lo;
       if constexpr (WALLS) {
         if (c < 0.0) la -= 2.0 * cwu;
         if (c > 0.0) lo -= 2.0 * cwu;
@@ -296,8 +297,7 @@ static void launch_pair(nat_ctx* ctx, const SedgArgs<T>& s, const CollideArgs<T>
 
 template <typename T>
 bool nat_sedg_pair_stage(nat_ctx* ctx, const SedgArgs<T>& s, const CollideArgs<T>& ca, int collide, int wm) {
-  // opposite directions are at most two arrays apart
-  if (!pair_offsets_fit(2, s.stride, sizeof(T))) return false;
+  if (nat_sedg_form(ctx) == 0) return false;
   const int Q = ctx->Q, P = ctx->p;
 #define NAT_SP(DD, QQ, PP)                              \
   if (Q == QQ && P == PP) {                             \

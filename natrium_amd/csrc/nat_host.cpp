@@ -41,6 +41,7 @@ int nat_comp_setup(nat_ctx* ctx);
 int nat_launch_sl_comp(nat_ctx* ctx, int write_macro);
 int nat_launch_collide_comp(nat_ctx* ctx);
 int nat_comp_form(const nat_ctx* ctx, int form);
+int nat_sedg_form(const nat_ctx* ctx, int form);
 
 namespace nat {
 
@@ -1354,6 +1355,8 @@ int nat_set_step_form(nat_ctx* ctx, int form) {
   bool ok = form == -1;
   if (ctx->desc.compressible)
     ok = ok || nat_comp_form(ctx, form);
+  else if (ctx->desc.scheme != NAT_SL)
+    ok = ok || nat_sedg_form(ctx, form);
   else
     return fail(ctx, NAT_ERR_ARG, "nat_set_step_form: the step of this context has no forms");
   if (form < -1 || !ok) return fail(ctx, NAT_ERR_ARG, "nat_set_step_form: no such form on this mesh");
@@ -1364,8 +1367,12 @@ int nat_set_step_form(nat_ctx* ctx, int form) {
 
 int nat_step_form(nat_ctx* ctx, int nsteps, int* form) {
   if (!form || nsteps < 1) return fail(ctx, NAT_ERR_ARG, "nat_step_form: a run of steps and a result are needed");
-  if (!ctx->desc.compressible) return fail(ctx, NAT_ERR_ARG, "nat_step_form: the step of this context has no forms");
-  *form = nat_comp_form(ctx, -1);
+  if (ctx->desc.compressible)
+    *form = nat_comp_form(ctx, -1);
+  else if (ctx->desc.scheme != NAT_SL)
+    *form = nat_sedg_form(ctx, -1);
+  else
+    return fail(ctx, NAT_ERR_ARG, "nat_step_form: the step of this context has no forms");
   return 0;
 }
 

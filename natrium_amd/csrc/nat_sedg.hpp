@@ -3,6 +3,8 @@
 #include "nat_collide.hpp"
 #include "nat_geom.hpp"
 
+int nat_sedg_form(const nat_ctx* ctx, int form = -1);
+
 namespace nat {
 
 template <typename T>
@@ -38,8 +40,9 @@ struct SedgShape {
 
 __device__ __forceinline__ void sedg_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// One RK5 stage of the upwind flux, two opposite directions at a time; false: the arrays are too
-// large for its 32-bit offsets and the caller takes the general stage kernel.
+// One RK5 stage of the upwind flux, two opposite directions at a time; false: the context's form is
+// another (the central flux, or arrays too large for 32-bit offsets) and the caller takes the
+// general stage kernel.
 template <typename T>
 bool nat_sedg_pair_stage(nat_ctx* ctx, const SedgArgs<T>& s, const CollideArgs<T>& ca, int collide, int wm);
 
