@@ -442,7 +442,7 @@ def main():
     bytes_per_launch = n_unique * 2 * Q * 4
     avg_launch_s = ms32 / 1e3 / args.steps
     achieved = bytes_per_launch / avg_launch_s / 1e9
-    long_run = args.steps >= 96  # on this mesh such runs take the collide-then-stream kernel
+    long_run = s32.step_form(args.steps) > 0  # the collide-then-stream kernel
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": read_traffic(("push_" if long_run else "") + workload),

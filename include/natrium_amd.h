@@ -249,6 +249,9 @@ int nat_set_general_form(nat_ctx* ctx, int form);
  * give bit-identical populations and fields and differ in the sizes they serve and in time.
  *   compressible: 1 reads a direction and its opposite at 32-bit offsets, 0 at 64-bit addresses
  *     (always available; the rule takes it for arrays of more than 4/3 GiB);
+ *   structured SL, runs of nsteps >= 2: 1 and 2 collide before they stream, with a small and a large
+ *     tile of cells per workgroup (p = 2-4, where that tile is built); 0 streams and collides in one
+ *     launch per step, as every single step does. The rule compares the tiles and the run length.
  *   SEDG: 1 works on opposite directions in pairs (upwind flux, arrays up to 4/3 GiB; the rule),
  *     0 on one direction at a time.
  * nat_set_step_form pins one (-1: the rule); NAT_ERR_ARG for a form this context does not have.

@@ -493,64 +493,19 @@ static int launch_push(nat_ctx* ctx, PushArgs<T> a, const CollideArgs<T>& ca, bo
   return 0;
 }
 
-// Tile of a context: 1 the small one, 2 the large one, 0 where k_sl_struct is faster. While the
-// small tiles leave CUs idle, a step lasts as long as one workgroup does, and less work per
-// workgroup wins; past a few workgroups per CU the share of nodes collided twice (NN over the
-// tile's nodes) and the length of the stored lines decide. k_sl_struct pays whole rounds of 256
-// tiles of 1024 nodes, so it is at its best where a mesh fills one (p=4 16^3, p=2 32^3 cells).
-// Cubic boxes, us per step in k_sl_struct / small / large tile (runs of 32 to 100 steps on a warm
-// card, one MI355X; -: no such tile):
-//   D3Q27 p=4 FP32   8^3 cells 14.1/ 9.2/11.8   12^3 17.4/14.3/13.8   16^3 20.8/25.0/20.3   30^3 221/171/139
-//             FP64   8^3       16.0/10.3/ -     11^3 21.3/20.0/ -     12^3 18.8/21.3/ -     16^3 28.4/40.7/ -
-//   D3Q19 p=4 FP32   8^3        9.4/ 7.0/ 8.4   12^3 11.0/10.0/ 9.1   16^3 13.4/18.5/14.0   24^3 47.8/56.2/42.2
-//             FP64   8^3       10.1/ 7.7/ -     11^3 14.3/11.8/ -     12^3 12.5/12.8/ -     16^3 18.5/24.3/ -
-//   D3Q19 p=3 FP32  16^3       13.9/ 8.7/ 8.7   21^3 32.5/16.7/14.8   32^3 66.5/41.1/37.9
-//             FP64  24^3       35.1/30.1/ -     28^3 57.5/39.9/ -     32^3 83.9/78.0/ -
-//   D3Q27 p=2 FP32  16^3       15.1/ 6.2/11.7   30^3 22.4/18.1/20.0   32^3 20.3/23.1/19.5   48^3 75.8/78.3/64.6
-//             FP64  16^3       16.3/ 6.6/ -     30^3 26.6/23.2/ -     32^3 26.6/29.1/ -     40^3 60.0/48.0/ -
-//   D3Q19 p=2 FP32  24^3       12.4/ 8.6/ 9.6   30^3 15.6/13.3/14.6   32^3 14.1/16.1/14.1   48^3 50.8/49.2/44.4
-//             FP64  30^3       17.9/16.2/ -     32^3 17.7/18.7/ -     40^3 39.0/32.6/ -     48^3 65.5/73.9/ -
-//   D2Q9  p=4 FP32   32^2       5.8/ 4.2/ 4.9   100^2 8.9/ 6.5/ 6.9   128^2 7.5/ 8.3/ 7.3   256^2 26.1/23.5/19.8
-//             FP64   32^2       6.2/ 4.3/ -     100^2 9.6/ 7.7/ -     128^2 9.5/10.5/ -
-//   D2Q9  p=2 FP32   64^2       5.7/ 3.3/ 4.0   128^2 5.6/ 4.0/ 4.1   256^2 7.6/ 7.7/ 7.0
-static int push_tile(const nat_ctx* ctx) {
-  const int64_t cells = (int64_t)ctx->desc.ncells[0] * ctx->desc.ncells[1] * (ctx->D == 3 ? ctx->desc.ncells[2] : 1);
-  if (ctx->D == 2) {
-    if (ctx->p == 2) return cells <= 16384 ? 1 : 2;
-    if (ctx->p == 3) return 1;
-    return cells <= 10240 ? 1 : (ctx->fp32 ? 2 : 0);
-  }
-  if (ctx->p == 2) {
-    if (ctx->fp32) return cells <= 28672 ? 1 : 2;
-    return cells <= 28672 || (cells > 32768 && cells < 65536) ? 1 : 0;
-  }
-  if (ctx->p == 3) return ctx->fp32 && cells > 8192 ? 2 : 1;
-  if (!ctx->fp32) return cells <= 1400 ? 1 : 0;
-  if (cells <= 1024) return 1;
-  return ctx->Q == 19 && cells > 3375 && cells <= 4096 ? 0 : 2;
-}
+// One instantiated tile.
+template <int D_, int Q_, int P_, int CX_, int CY_, int CZ_, int NT_, int S_, int WPE_>
+struct PushTile {
+  static constexpr int D = D_, Q = Q_, P = P_, CX = CX_, CY = CY_, CZ = CZ_, NT = NT_, S = S_, WPE = WPE_;
+};
 
-template <typename T>
-static int push_typed(nat_ctx* ctx, bool col) {
-  PushArgs<T> a{};
-  a.fin = (const T*)ctx->f[ctx->cur];
-  a.fout = (T*)ctx->f[1 - ctx->cur];
-  a.stride = ctx->stride;
-  for (int i = 0; i < 3; i++) a.n[i] = ctx->nu[i];
-  a.dir_bytes = (int)(ctx->stride * (int64_t)sizeof(T));
-  a.all_bytes = (unsigned)(ctx->stride * (int64_t)sizeof(T) * ctx->Q);
-  CollideArgs<T> ca{};
-  ca.omega = (T)(1.0 / ctx->tau);
-  ca.omega64 = 1.0 / ctx->tau;
-  ca.rho0 = (T)(ctx->fp32 ? (ctx->desc.rho0 > 0 ? ctx->desc.rho0 : 1.0) : 0.0);
-  ca.scaling = ctx->st.s;
-  ca.status = ctx->d_status;
-  ca.stab = ctx->stab_on();
-  const int Q = ctx->Q, P = ctx->p, tile = push_tile(ctx);
-  int rc = NAT_ERR_UNSUPPORTED;
+// Calls f(PushTile) for tile 1 (the small one) or 2 (the large one) of a stencil and order;
+// NAT_ERR_UNSUPPORTED: no such tile.
+template <typename T, typename F>
+static int push_dispatch(int tile, int Q, int P, F&& f) {
   // cells per workgroup, threads, parts per item, waves per SIMD the registers are held to
 #define NAT_P(tl, DD, QQ, PP, ...) \
-  if (tile == tl && Q == QQ && P == PP) rc = launch_push<DD, QQ, PP, T, __VA_ARGS__>(ctx, a, ca, col);
+  if (tile == tl && Q == QQ && P == PP) return f(PushTile<DD, QQ, PP, __VA_ARGS__>{});
 #define NAT_P3(tl, PP, ...)      \
   NAT_P(tl, 3, 19, PP, __VA_ARGS__) \
   NAT_P(tl, 3, 27, PP, __VA_ARGS__)
@@ -569,30 +524,141 @@ static int push_typed(nat_ctx* ctx, bool col) {
   }
 #undef NAT_P3
 #undef NAT_P
-  if (rc == 0) ctx->cur = 1 - ctx->cur;
-  return rc;
+  return NAT_ERR_UNSUPPORTED;
+}
+
+template <typename F>
+static int push_dispatch(const nat_ctx* ctx, int tile, F&& f) {
+  return ctx->fp32 ? push_dispatch<float>(tile, ctx->Q, ctx->p, f) : push_dispatch<double>(tile, ctx->Q, ctx->p, f);
+}
+
+// Cells of the workgroups that a tile takes for the mesh, those beyond a ragged one included.
+static int64_t push_cells(const nat_ctx* ctx, int tile) {
+  const int* N = ctx->desc.ncells;
+  int64_t cells = 0;
+  push_dispatch(ctx, tile, [&](auto tl) {
+    using L = decltype(tl);
+    const auto up = [](int n, int c) { return (int64_t)((n + c - 1) / c) * c; };
+    cells = up(N[0], L::CX) * up(N[1], L::CY) * (L::D == 3 ? up(N[2], L::CZ) : 1);
+    return 0;
+  });
+  return cells;
+}
+
+// Whether k_sl_struct's 16 x 8 x 8 tiles (3D, p = 2 and 4) fill one round of the CUs: more than
+// 5/6 of it, and no second one.
+static bool push_one_round(const nat_ctx* ctx) {
+  if (ctx->p == 3) return false;
+  const int64_t tiles = (int64_t)((ctx->nu[0] + 15) / 16) * ((ctx->nu[1] + 7) / 8) * ((ctx->nu[2] + 7) / 8);
+  return tiles <= ctx->n_cu && 6 * ctx->n_store >= 5 * (int64_t)ctx->n_cu * 1024;
+}
+
+// Tile of a context: 1 the small one, 2 the large one, 0 where k_sl_struct is faster. While the
+// small tiles leave CUs idle, a step lasts as long as one workgroup does, and less work per
+// workgroup wins; past a few workgroups per CU the share of nodes collided twice (NN over the
+// tile's nodes) and the length of the stored lines decide, and with them the cells that the tiles
+// hold beyond a ragged mesh: boxes a few cells thin stay with the small tile (2 x 32 x 25 cells,
+// D3Q27 p=4 FP32: 15.1 / 12.3 / 18.2). k_sl_struct pays whole rounds of a tile of 1024 nodes per
+// CU, so it is at its best where a mesh fills one (p=4 16^3, p=2 32^3 cells; from 5/6 of it on the
+// other form is 3-8% ahead or behind), and in FP64 its longer lines win at p=4, and beyond the
+// Infinity Cache at p=2.
+// Cubic boxes, us per step in k_sl_struct / small / large tile (runs of 32 to 100 steps on a warm
+// card, one MI355X; -: no such tile):
+//   D3Q27 p=4 FP32   8^3 cells 14.1/ 9.2/11.8   12^3 17.4/14.3/13.8   16^3 20.8/25.0/20.3   30^3 221/171/139
+//             FP64   8^3       16.0/10.3/ -     11^3 21.3/20.0/ -     12^3 18.8/21.3/ -     16^3 28.4/40.7/ -
+//   D3Q19 p=4 FP32   8^3        9.4/ 7.0/ 8.4   12^3 11.0/10.0/ 9.1   16^3 13.4/18.5/14.0   24^3 47.8/56.2/42.2
+//             FP64   8^3       10.1/ 7.7/ -     11^3 14.3/11.8/ -     12^3 12.5/12.8/ -     16^3 18.5/24.3/ -
+//   D3Q19 p=3 FP32  16^3       13.9/ 8.7/ 8.7   21^3 32.5/16.7/14.8   32^3 66.5/41.1/37.9
+//             FP64  24^3       35.1/30.1/ -     28^3 57.5/39.9/ -     32^3 83.9/78.0/ -
+//   D3Q27 p=2 FP32  16^3       15.1/ 6.2/11.7   30^3 22.4/18.1/20.0   32^3 20.3/23.1/19.5   48^3 75.8/78.3/64.6
+//             FP64  16^3       16.3/ 6.6/ -     30^3 26.6/23.2/ -     32^3 26.6/29.1/ -     40^3 60.0/48.0/ -
+//   D3Q19 p=2 FP32  24^3       12.4/ 8.6/ 9.6   30^3 15.6/13.3/14.6   32^3 14.1/16.1/14.1   48^3 50.8/49.2/44.4
+//             FP64  30^3       17.9/16.2/ -     32^3 17.7/18.7/ -     40^3 39.0/32.6/ -     48^3 65.5/73.9/ -
+//   D2Q9  p=4 FP32   32^2       5.8/ 4.2/ 4.9   100^2 8.9/ 6.5/ 6.9   128^2 7.5/ 8.3/ 7.3   256^2 26.1/23.5/19.8
+//             FP64   32^2       6.2/ 4.3/ -     100^2 9.6/ 7.7/ -     128^2 9.5/10.5/ -
+//   D2Q9  p=2 FP32   64^2       5.7/ 3.3/ 4.0   128^2 5.6/ 4.0/ 4.1   256^2 7.6/ 7.7/ 7.0
+static int push_tile(const nat_ctx* ctx) {
+  const int* N = ctx->desc.ncells;
+  const int64_t cells = (int64_t)N[0] * N[1] * (ctx->D == 3 ? N[2] : 1);
+  int tile;
+  if (ctx->D == 2) {
+    if (ctx->p == 4)
+      tile = cells <= 10240 ? 1 : (ctx->fp32 ? 2 : 0);
+    else
+      tile = ctx->p == 3 || cells <= 16384 ? 1 : 2;
+  } else if (ctx->p == 3) {
+    tile = ctx->fp32 && cells > 8192 ? 2 : 1;
+  } else if (ctx->p == 2) {
+    if (ctx->fp32)
+      tile = cells <= 28672 ? 1 : 2;
+    else
+      tile = cells < 65536 && !push_one_round(ctx) ? 1 : 0;
+  } else {
+    if (ctx->fp32)
+      tile = cells <= 1024 ? 1 : (ctx->Q == 19 && push_one_round(ctx) ? 0 : 2);
+    else
+      tile = cells <= 1400 ? 1 : 0;
+  }
+  return tile == 2 && 4 * push_cells(ctx, 2) > 5 * push_cells(ctx, 1) ? 1 : tile;
+}
+
+// The shortest run that takes the form. A run adds a launch and, with its collision, one more pass
+// over the populations: 2 us up to 3 MB of them, then about 0.3 us per MB (D3Q27 p=4 32^3 FP32,
+// 226 MB: 80 us), which the steps have to earn. Steps until they do, over 444 meshes, by what a
+// step gains (3D p=3: 20-60%; 2D p=4: 4-30%): up to 3 MB 2; 3D p=3 2.4, p=2 and 4 7; 2D p=2 and 3
+// 5, p=4 15. Where k_sl_struct's tiles fill one round the gain is 5% at most, and the first
+// hundred launches lose it (D3Q27 p=4 16^3 FP32, us per step in k_sl_struct / k_sl_push: runs of
+// 16 steps 21.8/23.3, 64 20.5/20.8, 128 20.6/20.0, 1000 20.9/19.9).
+static int push_min_steps(const nat_ctx* ctx) {
+  if (ctx->D == 3 && push_one_round(ctx)) return 96;
+  if (ctx->n_store * ctx->Q * (ctx->fp32 ? 4 : 8) <= 3000000) return 2;
+  if (ctx->D == 3) return ctx->p == 3 ? 3 : 8;
+  return ctx->p == 4 ? 16 : 6;
+}
+
+template <typename T>
+static int push_typed(nat_ctx* ctx, int tile, bool col) {
+  PushArgs<T> a{};
+  a.fin = (const T*)ctx->f[ctx->cur];
+  a.fout = (T*)ctx->f[1 - ctx->cur];
+  a.stride = ctx->stride;
+  for (int i = 0; i < 3; i++) a.n[i] = ctx->nu[i];
+  a.dir_bytes = (int)(ctx->stride * (int64_t)sizeof(T));
+  a.all_bytes = (unsigned)(ctx->stride * (int64_t)sizeof(T) * ctx->Q);
+  CollideArgs<T> ca{};
+  ca.omega = (T)(1.0 / ctx->tau);
+  ca.omega64 = 1.0 / ctx->tau;
+  ca.rho0 = (T)(ctx->fp32 ? (ctx->desc.rho0 > 0 ? ctx->desc.rho0 : 1.0) : 0.0);
+  ca.scaling = ctx->st.s;
+  ca.status = ctx->d_status;
+  ca.stab = ctx->stab_on();
+  return push_dispatch<T>(tile, ctx->Q, ctx->p, [&](auto tl) {
+    using L = decltype(tl);
+    return launch_push<L::D, L::Q, L::P, T, L::CX, L::CY, L::CZ, L::NT, L::S, L::WPE>(ctx, a, ca, col);
+  });
 }
 
 }  // namespace nat
 
-// Whether a run of nsteps steps of this context takes the collide-then-stream form: symmetric
-// one-dimensional tables at p = 2-4, populations within 32-bit buffer offsets, and a tile that is
-// faster than k_sl_struct's. On a mesh that fills one or two rounds of k_sl_struct's tiles exactly
-// (p=4 16^3, p=2 32^3) the two are close, and the run must be long: from an idle card the first
-// hundred launches are slower here (D3Q27 p=4 16^3 FP32, k_sl_struct / k_sl_push in us per step:
-// 16 steps 21.8/23.3, 64 20.5/20.8, 128 20.6/20.0, 1000 20.9/19.9).
-bool nat_push_eligible(const nat_ctx* ctx, int nsteps) {
-  if (nsteps < 2 || ctx->desc.scheme != NAT_SL || ctx->desc.compressible || ctx->backend != NAT_BACKEND_STRUCTURED ||
-      !ctx->ax_sym || !ctx->ax_w || ctx->p < 2 || ctx->p > 4 ||
-      ctx->stride * (ctx->fp32 ? 4 : 8) * ctx->Q >= (int64_t)0xffffffffu)
+// The tile exists for this context: a structured SL context with symmetric one-dimensional tables,
+// populations within 32-bit buffer offsets, and a tile of this (stencil, order, storage).
+bool nat_push_has(const nat_ctx* ctx, int tile) {
+  if (ctx->desc.scheme != NAT_SL || ctx->desc.compressible || ctx->backend != NAT_BACKEND_STRUCTURED || !ctx->ax_sym ||
+      !ctx->ax_w || ctx->stride * (ctx->fp32 ? 4 : 8) * ctx->Q >= (int64_t)0xffffffffu)
     return false;
-  const int tile = nat::push_tile(ctx);
-  const int64_t round = 256 * 1024;
-  const bool close = ctx->D == 3 && tile == 2 && ctx->n_store % round == 0 && ctx->n_store <= 2 * round;
-  return tile > 0 && (!close || nsteps >= 96);
+  return nat::push_dispatch(ctx, tile, [](auto) { return 0; }) == 0;
+}
+
+// Form of a run of nsteps steps: 0 k_sl_struct, else the tile of the collide-then-stream form.
+int nat_push_form(const nat_ctx* ctx, int nsteps) {
+  if (nsteps < 2 || !nat_push_has(ctx, 1)) return 0;
+  if (ctx->form_pref >= 0) return ctx->form_pref;
+  return nsteps >= nat::push_min_steps(ctx) ? nat::push_tile(ctx) : 0;
 }
 
 // One launch from f[cur] into f[1 - cur]: collide (when col) and stream.
-int nat_launch_sl_push(nat_ctx* ctx, bool col) {
-  return ctx->fp32 ? nat::push_typed<float>(ctx, col) : nat::push_typed<double>(ctx, col);
+int nat_launch_sl_push(nat_ctx* ctx, int tile, bool col) {
+  const int rc = ctx->fp32 ? nat::push_typed<float>(ctx, tile, col) : nat::push_typed<double>(ctx, tile, col);
+  if (rc == 0) ctx->cur = 1 - ctx->cur;
+  return rc;
 }

@@ -27,8 +27,9 @@ int nat_internal_pack_step(nat_ctx* const* ctxs, int n, int nsteps, hipStream_t 
 int nat_internal_autotune(nat_ctx* ctx, int nsteps, int* tile, double* best_us);
 int nat_internal_autotune_general(nat_ctx* ctx, int nsteps, int* tile, double* best_us);
 int nat_launch_sl_general(nat_ctx* ctx, int write_macro);
-bool nat_push_eligible(const nat_ctx* ctx, int nsteps);
-int nat_launch_sl_push(nat_ctx* ctx, bool col);
+bool nat_push_has(const nat_ctx* ctx, int tile);
+int nat_push_form(const nat_ctx* ctx, int nsteps);
+int nat_launch_sl_push(nat_ctx* ctx, int tile, bool col);
 int nat_launch_collide(nat_ctx* ctx, int init);
 int nat_launch_collide_step(nat_ctx* ctx, bool macro);
 int nat_launch_stabilize(nat_ctx* ctx);
@@ -1071,12 +1072,12 @@ int nat_stabilize(nat_ctx* ctx) {
 }
 
 // Runs of two steps or more of a structured context take the collide-then-stream form where it is
-// the faster (nat_push_eligible, k_sl_push.hip): n steps are one streaming launch, n - 1 launches
+// the faster (nat_push_form, k_sl_push.hip): n steps are one streaming launch, n - 1 launches
 // that collide and stream, and one collision, n + 1 in all. A single step would be two launches, and is one of the fused
 // stream-then-collide kernel instead.
-static int push_launch(nat_ctx* ctx, int n, bool col) {
+static int push_launch(nat_ctx* ctx, int tile, int n, bool col) {
   for (int s = 0; s < n; s++) {
-    TRY(nat_launch_sl_push(ctx, col));
+    TRY(nat_launch_sl_push(ctx, tile, col));
     ctx->time += ctx->dt;
   }
   return 0;
@@ -1084,9 +1085,9 @@ static int push_launch(nat_ctx* ctx, int n, bool col) {
 
 static int step_launch(nat_ctx* ctx, int nsteps, bool macro_last = true) {
   if (!ctx->assembled) return fail(ctx, NAT_ERR_STATE, "operator not assembled");
-  if (nat_push_eligible(ctx, nsteps)) {
-    TRY(push_launch(ctx, 1, false));
-    TRY(push_launch(ctx, nsteps - 1, true));
+  if (const int tile = nat_push_form(ctx, nsteps)) {
+    TRY(push_launch(ctx, tile, 1, false));
+    TRY(push_launch(ctx, tile, nsteps - 1, true));
     return nat_launch_collide_step(ctx, macro_last);
   }
   for (int s = 0; s < nsteps; s++) {
@@ -1152,16 +1153,17 @@ extern "C++" int nat_internal_capture(nat_ctx* ctx, int nsteps, bool macro_last,
 
 static int step_enqueue(nat_ctx* ctx, int nsteps) {
   int left = nsteps;
-  const bool push = ctx->assembled && nat_push_eligible(ctx, nsteps);
+  const int tile = ctx->assembled ? nat_push_form(ctx, nsteps) : 0;
+  const bool push = tile > 0;
   // collide-then-stream: the streaming of the first step, then graphs of (collide; stream)
-  if (push) TRY(push_launch(ctx, 1, false));
+  if (push) TRY(push_launch(ctx, tile, 1, false));
   // the last step writes the macroscopic fields and always runs as a plain launch
   while (ctx->use_graphs && left - 1 >= kGraphSteps) {
     const int par = ctx->cur + (push ? 2 : 0);
     if (!ctx->gexec[par]) {
       hipGraph_t g = nullptr;
       TRY(capture(ctx, &g, [&] {
-        return push ? push_launch(ctx, kGraphSteps, true) : step_launch(ctx, kGraphSteps, false);
+        return push ? push_launch(ctx, tile, kGraphSteps, true) : step_launch(ctx, kGraphSteps, false);
       }));
       ctx->graph[par] = g;
       NAT_HIP(hipGraphInstantiate(&ctx->gexec[par], g, nullptr, nullptr, 0));
@@ -1171,7 +1173,7 @@ static int step_enqueue(nat_ctx* ctx, int nsteps) {
     left -= kGraphSteps;
   }
   if (push) {
-    TRY(push_launch(ctx, left - 1, true));
+    TRY(push_launch(ctx, tile, left - 1, true));
     return nat_launch_collide_step(ctx, true);
   }
   return step_launch(ctx, left);
@@ -1357,6 +1359,8 @@ int nat_set_step_form(nat_ctx* ctx, int form) {
     ok = ok || nat_comp_form(ctx, form);
   else if (ctx->desc.scheme != NAT_SL)
     ok = ok || nat_sedg_form(ctx, form);
+  else if (ctx->backend == NAT_BACKEND_STRUCTURED)
+    ok = ok || form == 0 || nat_push_has(ctx, form);
   else
     return fail(ctx, NAT_ERR_ARG, "nat_set_step_form: the step of this context has no forms");
   if (form < -1 || !ok) return fail(ctx, NAT_ERR_ARG, "nat_set_step_form: no such form on this mesh");
@@ -1371,6 +1375,8 @@ int nat_step_form(nat_ctx* ctx, int nsteps, int* form) {
     *form = nat_comp_form(ctx, -1);
   else if (ctx->desc.scheme != NAT_SL)
     *form = nat_sedg_form(ctx, -1);
+  else if (ctx->backend == NAT_BACKEND_STRUCTURED)
+    *form = nat_push_form(ctx, nsteps);
   else
     return fail(ctx, NAT_ERR_ARG, "nat_step_form: the step of this context has no forms");
   return 0;

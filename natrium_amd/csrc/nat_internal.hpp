@@ -197,7 +197,7 @@ struct nat_ctx {
   int* ax_off = nullptr;  // [3][MAXSHIFT][MAXP] source cell offsets
   bool ax_sym = false;    // tables equal on all axes and mirror symmetric in the shift sign
   int tile_pref = -1;     // structured tile: -1 size heuristic, 0 large tile, 1 small tile (autotuner)
-  int form_pref = -1;     // step kernel form of a compressible or SEDG context (nat_set_step_form): -1 the rule
+  int form_pref = -1;     // step kernel form (nat_set_step_form): -1 the rule
   int gen_pref = -1;      // general SL FP32 3D kernel: -1 grid-size rule, 0 eight waves per block, 1 sixteen (autotuner)
   int sid[nat::MAXQ][3] = {};
   int off_lo[3][nat::MAXSHIFT] = {}, off_hi[3][nat::MAXSHIFT] = {};
