@@ -231,7 +231,8 @@ int nat_step_packed(nat_ctx* const* ctxs, int n, int nsteps);
  * contexts of the same kernel instantiation and mesh size (which then skip the timing). The
  * timing launches write only the idle population buffer: populations, fields and time are
  * unchanged, and results do not depend on the shape. SL contexts (not compressible):
- *   structured backend: the tiles; tile receives the chosen (x, y, z) extents;
+ *   structured backend: the tiles of the kernel that single and packed steps take (tile receives the
+ *     chosen (x, y, z) extents) and the forms of a run of steps (nat_step_form tells the choice);
  *   general backend: with FP32 storage in 3D the eight-wave and the sixteen-wave form of a block
  *     of DoFs (the latter by default up to 5/2 blocks per CU); tile receives the chosen form's
  *     (DoFs per block, waves per SIMD it is built for, z-planes of source rows loaded

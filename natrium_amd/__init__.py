@@ -391,8 +391,9 @@ class Solver:
 
     def autotune(self, nsteps=10):
         """Time the SL kernel's launch shapes on this mesh and keep the fastest (nat_autotune);
-        returns the chosen tile (structured backend) or (DoFs per block, waves per SIMD,
-        z-planes in flight) of the chosen form (general backend)."""
+        returns the chosen tile of single steps (structured backend; step_form tells the form of
+        a run) or (DoFs per block, waves per SIMD, z-planes in flight) of the chosen form
+        (general backend)."""
         t = (ctypes.c_int * 3)()
         self._check(lib().nat_autotune(self._h, int(nsteps), t))
         return tuple(t)

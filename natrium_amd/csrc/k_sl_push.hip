@@ -653,12 +653,17 @@ bool nat_push_has(const nat_ctx* ctx, int tile) {
 int nat_push_form(const nat_ctx* ctx, int nsteps) {
   if (nsteps < 2 || !nat_push_has(ctx, 1)) return 0;
   if (ctx->form_pref >= 0) return ctx->form_pref;
-  return nsteps >= nat::push_min_steps(ctx) ? nat::push_tile(ctx) : 0;
+  if (nsteps < nat::push_min_steps(ctx)) return 0;
+  return ctx->push_pref >= 0 ? ctx->push_pref : nat::push_tile(ctx);
 }
 
-// One launch from f[cur] into f[1 - cur]: collide (when col) and stream.
-int nat_launch_sl_push(nat_ctx* ctx, int tile, bool col) {
+// The rule's form of a long run.
+int nat_push_tile(const nat_ctx* ctx) { return nat_push_has(ctx, 1) ? nat::push_tile(ctx) : 0; }
+
+// One launch from f[cur] into f[1 - cur]: collide (when col) and stream. advance: the written
+// buffer becomes the current one.
+int nat_launch_sl_push(nat_ctx* ctx, int tile, bool col, bool advance) {
   const int rc = ctx->fp32 ? nat::push_typed<float>(ctx, tile, col) : nat::push_typed<double>(ctx, tile, col);
-  if (rc == 0) ctx->cur = 1 - ctx->cur;
+  if (rc == 0 && advance) ctx->cur = 1 - ctx->cur;
   return rc;
 }

@@ -553,10 +553,28 @@ struct TuneKey {
   }
 };
 std::mutex g_tune_mutex;
-std::map<TuneKey, int> g_tune_cache;  // winning tile preference per (instantiation, mesh)
+struct Tuned {
+  int tile;  // k_sl_struct's tile (nat_ctx::tile_pref)
+  int form;  // form of a run (nat_ctx::push_pref)
+};
+std::map<TuneKey, Tuned> g_tune_cache;  // winners per (instantiation, mesh)
 
-// device time of nsteps launches of the step kernel with the context's current tile choice;
-// each reads the current buffer and writes the other one without advancing the state
+// device time of nsteps launches, each reading the current buffer and writing the other one
+// without advancing the state
+template <typename F>
+int time_launches(nat_ctx* ctx, int nsteps, hipEvent_t e0, hipEvent_t e1, float* ms, F&& launch) {
+  for (int s = 0; s < 2; s++)
+    if (int rc = launch()) return rc;
+  NAT_HIP(hipEventRecord(e0, ctx->stream));
+  for (int s = 0; s < nsteps; s++)
+    if (int rc = launch()) return rc;
+  NAT_HIP(hipEventRecord(e1, ctx->stream));
+  NAT_HIP(hipEventSynchronize(e1));
+  NAT_HIP(hipEventElapsedTime(ms, e0, e1));
+  return 0;
+}
+
+// the same of the step kernel with the context's current tile choice
 template <typename T>
 int time_tile(nat_ctx* ctx, int nsteps, hipEvent_t e0, hipEvent_t e1, float* ms) {
   nat::StructArgs<T> a;
@@ -564,26 +582,21 @@ int time_tile(nat_ctx* ctx, int nsteps, hipEvent_t e0, hipEvent_t e1, float* ms)
   if (int rc = nat::make_args<T>(ctx, ctx->cur, a, ca)) return rc;
   ca.rho = nullptr;
   ca.u = nullptr;
-  nat::StructMode md;
-  for (int s = 0; s < 2; s++)
-    if (int rc = nat::dispatch_struct<T>(ctx, a, ca, 0, md)) return rc;
-  NAT_HIP(hipEventRecord(e0, ctx->stream));
-  for (int s = 0; s < nsteps; s++)
-    if (int rc = nat::dispatch_struct<T>(ctx, a, ca, 0, md)) return rc;
-  NAT_HIP(hipEventRecord(e1, ctx->stream));
-  NAT_HIP(hipEventSynchronize(e1));
-  NAT_HIP(hipEventElapsedTime(ms, e0, e1));
-  return 0;
+  const nat::StructMode md;
+  return time_launches(ctx, nsteps, e0, e1, ms, [&] { return nat::dispatch_struct<T>(ctx, a, ca, 0, md); });
 }
 
 }  // namespace
 
-// Tile shape of the structured step kernel picked by measurement: every tile instantiated for
-// the context's (stencil, order) is timed for nsteps steps on the context's own mesh (the
-// launches write the idle ping-pong buffer; populations, fields and time stay as they were),
-// and the fastest is kept for this context and, process-wide, for every later context of the
-// same instantiation and mesh size, which then skips the timing. Results do not depend on the
-// tile: each node's interpolation and collision run the same arithmetic in any tile.
+// Launch shapes of the structured step picked by measurement: every tile of k_sl_struct
+// instantiated for the context's (stencil, order), and every tile of the collide-then-stream form
+// of runs, is timed for nsteps steps on the context's own mesh (the launches write the idle
+// ping-pong buffer; populations, fields and time stay as they were). The fastest tile of
+// k_sl_struct, and the form of a run, are kept for this context and, process-wide, for every later
+// context of the same instantiation and mesh size, which then skips the timing. A run takes another
+// form than its rule says where that is 5% faster: small meshes are timed at the rate of single
+// launches here, which hides differences that a captured run shows. Results do not depend on any
+// of it: each node's interpolation and collision run the same arithmetic in every shape.
 int nat_internal_autotune(nat_ctx* ctx, int nsteps, int* tile, double* best_us) {
   if (ctx->desc.scheme != NAT_SL || ctx->desc.compressible || ctx->backend != NAT_BACKEND_STRUCTURED) {
     ctx->err = "nat_autotune: the autotuner serves the structured and general SL backends";
@@ -596,7 +609,8 @@ int nat_internal_autotune(nat_ctx* ctx, int nsteps, int* tile, double* best_us) 
     std::lock_guard<std::mutex> lk(g_tune_mutex);
     auto it = g_tune_cache.find(key);
     if (it != g_tune_cache.end()) {
-      ctx->tile_pref = it->second;
+      ctx->tile_pref = it->second.tile;
+      ctx->push_pref = it->second.form;
       return nat_launch_sl_struct_tile(ctx, tile);
     }
   }
@@ -623,6 +637,19 @@ int nat_internal_autotune(nat_ctx* ctx, int nsteps, int* tile, double* best_us) 
       best_ms = ms;
     }
   }
+  const int rule = nat_push_tile(ctx);
+  int form = 0;
+  float form_ms = best_ms * (rule == 0 ? 0.95f : 1.f);
+  for (int tile = 1; tile <= 2 && !rc; tile++) {
+    if (!nat_push_has(ctx, tile)) continue;
+    float ms = 0;
+    rc = time_launches(ctx, nsteps, e0, e1, &ms, [&] { return nat_launch_sl_push(ctx, tile, true, false); });
+    if (tile == rule) ms *= 0.95f;
+    if (!rc && ms < form_ms) {
+      form = tile;
+      form_ms = ms;
+    }
+  }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (rc) {
@@ -630,10 +657,11 @@ int nat_internal_autotune(nat_ctx* ctx, int nsteps, int* tile, double* best_us) 
     return rc;
   }
   ctx->tile_pref = best;
+  ctx->push_pref = form;
   if (best_us) *best_us = 1e3 * best_ms / nsteps;
   {
     std::lock_guard<std::mutex> lk(g_tune_mutex);
-    g_tune_cache[key] = best;
+    g_tune_cache[key] = {best, form};
   }
   return nat_launch_sl_struct_tile(ctx, tile);
 }

@@ -27,9 +27,7 @@ int nat_internal_pack_step(nat_ctx* const* ctxs, int n, int nsteps, hipStream_t 
 int nat_internal_autotune(nat_ctx* ctx, int nsteps, int* tile, double* best_us);
 int nat_internal_autotune_general(nat_ctx* ctx, int nsteps, int* tile, double* best_us);
 int nat_launch_sl_general(nat_ctx* ctx, int write_macro);
-bool nat_push_has(const nat_ctx* ctx, int tile);
 int nat_push_form(const nat_ctx* ctx, int nsteps);
-int nat_launch_sl_push(nat_ctx* ctx, int tile, bool col);
 int nat_launch_collide(nat_ctx* ctx, int init);
 int nat_launch_collide_step(nat_ctx* ctx, bool macro);
 int nat_launch_stabilize(nat_ctx* ctx);
@@ -1077,7 +1075,7 @@ int nat_stabilize(nat_ctx* ctx) {
 // stream-then-collide kernel instead.
 static int push_launch(nat_ctx* ctx, int tile, int n, bool col) {
   for (int s = 0; s < n; s++) {
-    TRY(nat_launch_sl_push(ctx, tile, col));
+    TRY(nat_launch_sl_push(ctx, tile, col, true));
     ctx->time += ctx->dt;
   }
   return 0;

@@ -197,6 +197,7 @@ struct nat_ctx {
   int* ax_off = nullptr;  // [3][MAXSHIFT][MAXP] source cell offsets
   bool ax_sym = false;    // tables equal on all axes and mirror symmetric in the shift sign
   int tile_pref = -1;     // structured tile: -1 size heuristic, 0 large tile, 1 small tile (autotuner)
+  int push_pref = -1;     // form of a structured run: -1 the rule, 0 k_sl_struct, 1 and 2 k_sl_push's tile (autotuner)
   int form_pref = -1;     // step kernel form (nat_set_step_form): -1 the rule
   int gen_pref = -1;      // general SL FP32 3D kernel: -1 grid-size rule, 0 eight waves per block, 1 sixteen (autotuner)
   int sid[nat::MAXQ][3] = {};
@@ -212,6 +213,11 @@ struct nat_ctx {
 
   std::string err;
 };
+
+// Collide-then-stream launches of structured runs (k_sl_push.hip)
+bool nat_push_has(const nat_ctx* ctx, int tile);
+int nat_push_tile(const nat_ctx* ctx);
+int nat_launch_sl_push(nat_ctx* ctx, int tile, bool col, bool advance);
 
 // error helpers
 #define NAT_HIP(call)                                                           \

@@ -112,3 +112,26 @@ def test_general_contexts_keep_their_own_setter():
                    backend="general")
     with pytest.raises(nat.NatError):
         g.set_step_form(0)
+
+
+def test_autotuned_form_is_what_a_run_takes():
+    """A box on which the rule keeps the fused kernel and the other form is 30% faster: the tuner
+    moves its runs, a second context of the size gets the choice without timing, and neither the
+    state at the time nor the results depend on it."""
+    N, p = [44, 44, 44], 2
+    a, b, c = (_solver("D3Q19", N, p, "fp64", init=init) for init in (True, True, False))
+    assert a.step_form(1000) == 0
+    f0, t0 = a.download_f(), a.time
+    tile = a.autotune(10)
+    assert tile == a.struct_tile()
+    np.testing.assert_array_equal(a.download_f(), f0)
+    assert a.time == t0
+    assert a.step_form(1000) == 1 and a.step_form(1) == 0 and b.step_form(1000) == 0
+    assert c.autotune(10) == tile and c.step_form(1000) == 1
+    a.step(9)
+    b.step(9)
+    np.testing.assert_array_equal(a.download_f(), b.download_f())
+    a.set_step_form(0)  # a pinned form stands above the tuned one
+    assert a.step_form(1000) == 0
+    a.set_step_form(-1)
+    assert a.step_form(1000) == 1
