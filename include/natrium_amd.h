@@ -254,7 +254,10 @@ int nat_set_general_form(nat_ctx* ctx, int form);
  *     tile of cells per workgroup (p = 2-4, where that tile is built); 0 streams and collides in one
  *     launch per step, as every single step does. The rule compares the tiles and the run length.
  *   SEDG: 1 works on opposite directions in pairs (upwind flux, arrays up to 4/3 GiB; the rule),
- *     0 on one direction at a time.
+ *     0 on one direction at a time;
+ *   general SL: 1 sixteen waves per block of DoFs (the rule up to 5/2 blocks per CU), 0 two per 64
+ *     DoFs; a choice here stands above nat_set_general_form's and the autotuner's, and serves all
+ *     storage precisions and dimensions.
  * nat_set_step_form pins one (-1: the rule); NAT_ERR_ARG for a form this context does not have.
  * nat_step_form returns the form a run of nsteps >= 1 steps takes. */
 int nat_set_step_form(nat_ctx* ctx, int form);

@@ -548,11 +548,12 @@ static int launch_general_shape(nat_ctx* ctx, const GeneralArgs<T>& a, const Col
   return 0;
 }
 
-// The wide form when the autotuner or the caller chose it (FP32 3D) or, by default, up to 5/2
+// The wide form when the caller chose it, or the autotuner (FP32 3D), or by default up to 5/2
 // blocks per CU, where the other form leaves a SIMD with few waves (figures at GeneralShape; FP32
 // 460 blocks: equal; 887: 73 us against 74; FP64 516 blocks: 11.4 against 9.5; 920: 41 against 44).
 template <int D, int Q, int P, typename T>
 static bool wide_form(const nat_ctx* ctx, int64_t n) {
+  if (ctx->form_pref >= 0) return ctx->form_pref == 1;
   if (sizeof(T) == 4 && D == 3 && ctx->gen_pref >= 0) return ctx->gen_pref == 1;
   constexpr int bs = GeneralShape<D, Q, P, T, true>::bs;
   return 2 * ((n + bs - 1) / bs) <= 5 * (int64_t)ctx->n_cu;
@@ -690,6 +691,17 @@ std::mutex g_gen_mutex;
 std::map<GenKey, int> g_gen_cache;
 
 }  // namespace
+
+// Form of the step: 0 W = 2 G waves per block, 1 the wide form (-1: no kernel for the context).
+int nat_general_form(nat_ctx* ctx) {
+  int form = -1;
+  nat::dispatch_dqp(ctx, [&](auto d, auto q, auto p) {
+    constexpr int D = decltype(d)::value, Q = decltype(q)::value, P = decltype(p)::value;
+    form = ctx->fp32 ? nat::wide_form<D, Q, P, float>(ctx, ctx->n_dofs) : nat::wide_form<D, Q, P, double>(ctx, ctx->n_dofs);
+    return 0;
+  });
+  return form;
+}
 
 int nat_launch_sl_general(nat_ctx* ctx, int write_macro) {
   const int rc = general_launch(ctx, write_macro);

@@ -27,6 +27,7 @@ int nat_internal_pack_step(nat_ctx* const* ctxs, int n, int nsteps, hipStream_t 
 int nat_internal_autotune(nat_ctx* ctx, int nsteps, int* tile, double* best_us);
 int nat_internal_autotune_general(nat_ctx* ctx, int nsteps, int* tile, double* best_us);
 int nat_launch_sl_general(nat_ctx* ctx, int write_macro);
+int nat_general_form(nat_ctx* ctx);
 int nat_push_form(const nat_ctx* ctx, int nsteps);
 int nat_launch_collide(nat_ctx* ctx, int init);
 int nat_launch_collide_step(nat_ctx* ctx, bool macro);
@@ -1352,15 +1353,15 @@ int nat_set_general_form(nat_ctx* ctx, int form) {
 }
 
 int nat_set_step_form(nat_ctx* ctx, int form) {
-  bool ok = form == -1;
+  bool ok = form == -1 || form == 0;
   if (ctx->desc.compressible)
     ok = ok || nat_comp_form(ctx, form);
   else if (ctx->desc.scheme != NAT_SL)
     ok = ok || nat_sedg_form(ctx, form);
   else if (ctx->backend == NAT_BACKEND_STRUCTURED)
-    ok = ok || form == 0 || nat_push_has(ctx, form);
+    ok = ok || nat_push_has(ctx, form);
   else
-    return fail(ctx, NAT_ERR_ARG, "nat_set_step_form: the step of this context has no forms");
+    ok = ok || form == 1;
   if (form < -1 || !ok) return fail(ctx, NAT_ERR_ARG, "nat_set_step_form: no such form on this mesh");
   if (form != ctx->form_pref) nat_drop_graphs(ctx);  // captured steps hold the other form's launches
   ctx->form_pref = form;
@@ -1376,7 +1377,7 @@ int nat_step_form(nat_ctx* ctx, int nsteps, int* form) {
   else if (ctx->backend == NAT_BACKEND_STRUCTURED)
     *form = nat_push_form(ctx, nsteps);
   else
-    return fail(ctx, NAT_ERR_ARG, "nat_step_form: the step of this context has no forms");
+    *form = nat_general_form(ctx);
   return 0;
 }
 

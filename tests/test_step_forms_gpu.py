@@ -106,14 +106,6 @@ def test_rule(stencil, N, p, precision, lines):
         assert g.step_form(1000) == (0 if form == 0 else lines[-1][1])
 
 
-def test_general_contexts_keep_their_own_setter():
-    N = [4, 4]
-    g = nat.Solver("D2Q9", 2, N, box_vertices(2, N, [0, 0], [1, 1]), cartesian=False, scaling=20.0, viscosity=0.01,
-                   backend="general")
-    with pytest.raises(nat.NatError):
-        g.set_step_form(0)
-
-
 def test_autotuned_form_is_what_a_run_takes():
     """A box on which the rule keeps the fused kernel and the other form is 30% faster: the tuner
     moves its runs, a second context of the size gets the choice without timing, and neither the
