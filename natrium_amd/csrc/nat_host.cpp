@@ -1154,20 +1154,24 @@ static int step_enqueue(nat_ctx* ctx, int nsteps) {
   int left = nsteps;
   const int tile = ctx->assembled ? nat_push_form(ctx, nsteps) : 0;
   const bool push = tile > 0;
+  const bool graphs = ctx->use_graphs && nsteps - 1 >= kGraphSteps;
   // collide-then-stream: the streaming of the first step, then graphs of (collide; stream)
+  const int start = push ? 1 - ctx->cur : ctx->cur;  // buffer that the graphs start from
+  const int slot = start + (push ? 2 : 0);
+  if (graphs && !ctx->gexec[slot]) {
+    // before the first launch: where a graph cannot be made, the populations are still whole steps
+    hipGraph_t g = nullptr;
+    TRY(capture(ctx, &g, [&] {
+      ctx->cur = start;
+      return push ? push_launch(ctx, tile, kGraphSteps, true) : step_launch(ctx, kGraphSteps, false);
+    }));
+    ctx->graph[slot] = g;
+    NAT_HIP(hipGraphInstantiate(&ctx->gexec[slot], g, nullptr, nullptr, 0));
+  }
   if (push) TRY(push_launch(ctx, tile, 1, false));
   // the last step writes the macroscopic fields and always runs as a plain launch
-  while (ctx->use_graphs && left - 1 >= kGraphSteps) {
-    const int par = ctx->cur + (push ? 2 : 0);
-    if (!ctx->gexec[par]) {
-      hipGraph_t g = nullptr;
-      TRY(capture(ctx, &g, [&] {
-        return push ? push_launch(ctx, tile, kGraphSteps, true) : step_launch(ctx, kGraphSteps, false);
-      }));
-      ctx->graph[par] = g;
-      NAT_HIP(hipGraphInstantiate(&ctx->gexec[par], g, nullptr, nullptr, 0));
-    }
-    NAT_HIP(hipGraphLaunch(ctx->gexec[par], ctx->stream));
+  while (graphs && left - 1 >= kGraphSteps) {
+    NAT_HIP(hipGraphLaunch(ctx->gexec[slot], ctx->stream));
     for (int st = 0; st < kGraphSteps; st++) ctx->time += ctx->dt;  // as step by step
     left -= kGraphSteps;
   }
