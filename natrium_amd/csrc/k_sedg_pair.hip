@@ -14,7 +14,8 @@
 //     with nothing to read has an offset out of range, which loads nothing and gives 0;
 //   - both values of a pair meet in LDS as one double2, with one barrier and one read of the
 //     derivative matrix for the two.
-// us per step (5 stages), one direction at a time with branches -> pairs, periodic:
+// us per step (5 stages), one direction at a time with branches -> pairs, periodic (before the face
+// sums were selected for the upwind one, which costs 0-3%):
 //   D3Q19 p=3 FP32   8^3 106 -> 38    24^3  600 -> 270   40^3 3331 -> 1482
 //   D3Q19 p=3 FP64   8^3  88 -> 38    24^3  737 -> 557   40^3 3191 -> 2435
 //   D3Q27 p=3        24^3 FP32 973 -> 454, FP64 1028 -> 801

@@ -104,8 +104,9 @@ constexpr int opposite(int i) {
 
 // FP64 BGK collision of populations held in storage precision, every relaxed population
 // handed to store(std::integral_constant<int, i>, value) as soon as it is formed. The
-// equilibrium of each opposite pair (i, i') comes from shared even and odd parts: f_eq(i/i') = w (E +- O), E = drho + rho (ue^2/2 - 3u.u/2),
-// O = rho ue (the direction-by-direction form of Equilibria.h:66-83 up to FP64 rounding).
+// equilibrium of each opposite pair (i, i') comes from shared even and odd parts:
+// f_eq(i/i') = w (E +- O), E = drho + rho (ue^2/2 - 3u.u/2), O = rho ue (the
+// direction-by-direction form of Equilibria.h:66-83 up to FP64 rounding).
 // Every step kernel and the collision-only pass use this one function, so their results
 // agree bit for bit.
 //

@@ -311,11 +311,11 @@ void dg_points(const nat_ctx* c, std::vector<double>& xyz) {
       }
 }
 
-// Elements between the arrays of two directions: whole 512-byte lines, and in FP32 or 2D not a
-// multiple of 1 MiB, which puts the same node of all directions on one memory channel (2,097,152
-// nodes in FP32, D3Q27 p = 4: 180 us per step at 8 MiB, 147 with 16,640 bytes more; 512^2 nodes in
-// FP64, D2Q9 p = 2: 9.5 -> 8.9). FP64 in 3D gains nothing (D3Q27 p = 4, 64^3 nodes: 26.95 -> 27.15,
-// 128^3: 268 -> 270).
+// Elements between the arrays of two directions: whole 512-byte lines (256 where padded), and in
+// FP32 or 2D not a multiple of 1 MiB, which puts the same node of all directions on one memory
+// channel (2,097,152 nodes in FP32, D3Q27 p = 4: 180 us per step at 8 MiB, 147 with 16,640 bytes
+// more; 512^2 nodes in FP64, D2Q9 p = 2: 9.5 -> 8.9). FP64 in 3D gains nothing (D3Q27 p = 4, 64^3
+// nodes: 26.95 -> 27.15, 128^3: 268 -> 270).
 int64_t pop_stride(int64_t n, int64_t es, int D) {
   const int64_t s = (n + 127) / 128 * 128;
   return (es == 4 || D == 2) && s * es % (1 << 20) == 0 ? s + 16640 / es : s;
@@ -1072,8 +1072,8 @@ int nat_stabilize(nat_ctx* ctx) {
 
 // Runs of two steps or more of a structured context take the collide-then-stream form where it is
 // the faster (nat_push_form, k_sl_push.hip): n steps are one streaming launch, n - 1 launches
-// that collide and stream, and one collision, n + 1 in all. A single step would be two launches, and is one of the fused
-// stream-then-collide kernel instead.
+// that collide and stream, and one collision, n + 1 in all. A single step would be two launches,
+// and is one of the fused stream-then-collide kernel instead.
 static int push_launch(nat_ctx* ctx, int tile, int n, bool col) {
   for (int s = 0; s < n; s++) {
     TRY(nat_launch_sl_push(ctx, tile, col, true));
